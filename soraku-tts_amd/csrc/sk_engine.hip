@@ -47,10 +47,14 @@ hipError_t dalloc(T** p, size_t n) {
   return hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T) + 256);
 }
 
-// Activation buffers of the batched prefill, M = packed prefix tokens.
+// Activation buffers of the batched prefill, M = packed prefix tokens.  Xn,
+// ATT and ACT hold FP32 or, with BF16 weights, hi and lo BF16 planes (the same
+// bytes).  QKV holds the q/k/v projection's K slices and is followed by Q; the
+// O and down projections' slices (P) use QKV and Q, which are dead by then.
 struct PrefillBufs {
   float *X = nullptr, *Xn = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *ACT = nullptr;
   int *tok_row = nullptr, *tok_pos = nullptr;
+  int qkv_split = 1, p_split = 1;   // most K slices that fit
 };
 
 // Scratch of sk_prefill_run_noalloc: the prefill's activation buffers for up
@@ -77,29 +81,39 @@ hipError_t scratch_ptr(int device, void** out) {
   return hipSuccess;
 }
 
-// Bytes of PrefillBufs for M tokens, each buffer 256-byte aligned.
-size_t prefill_bytes(const sk_config& c, int nqkv, size_t M) {
-  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Bytes of PrefillBufs for M tokens, each buffer 256-byte aligned, and where
+// QKV's share goes: one slice, or for few tokens (whose GEMMs need their K cut
+// to fill the GPU) up to 4 MB of slices, as long as that alone does not push
+// the prefill past the scratch of sk_prefill_run_noalloc.
+struct PrefillSizes { size_t qkv, total; };
+PrefillSizes prefill_sizes(const sk_config& c, int nqkv, size_t M) {
   const size_t hq = (size_t)c.n_q_heads * c.head_dim;
-  return up(M * c.d_model * 4) * 2 + up(M * nqkv * 4) + up(M * hq * 4) * 2 + up(M * c.trunk_inter * 4) +
-         up(M * 4) * 2;
+  const size_t rest = up256(M * c.d_model * 4) * 2 + up256(M * hq * 4) * 2 + up256(M * c.trunk_inter * 4) +
+                      up256(M * 4) * 2;
+  const size_t one = up256(M * nqkv * 4), room = SK_NOALLOC_SCRATCH_BYTES;
+  size_t qkv = std::max(one, std::min<size_t>(4u << 20, rest < room ? (room - rest) & ~(size_t)255 : 0));
+  return PrefillSizes{qkv, rest + qkv};
 }
 
-// Carves PrefillBufs for M tokens out of `base` (prefill_bytes(M) bytes).
+// Carves PrefillBufs for M tokens out of `base` (prefill_sizes(M).total bytes).
 PrefillBufs carve_prefill(const sk_config& c, int nqkv, size_t M, void* base) {
-  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t hq = (size_t)c.n_q_heads * c.head_dim;
+  const PrefillSizes z = prefill_sizes(c, nqkv, M);
   char* p = static_cast<char*>(base);
-  auto take = [&](size_t bytes) { char* q = p; p += up(bytes); return q; };
+  auto take = [&](size_t bytes) { char* q = p; p += up256(bytes); return q; };
   PrefillBufs b;
   b.X = reinterpret_cast<float*>(take(M * c.d_model * 4));
   b.Xn = reinterpret_cast<float*>(take(M * c.d_model * 4));
-  b.QKV = reinterpret_cast<float*>(take(M * nqkv * 4));
+  b.QKV = reinterpret_cast<float*>(take(z.qkv));
   b.Q = reinterpret_cast<float*>(take(M * hq * 4));
   b.ATT = reinterpret_cast<float*>(take(M * hq * 4));
   b.ACT = reinterpret_cast<float*>(take(M * c.trunk_inter * 4));
   b.tok_row = reinterpret_cast<int*>(take(M * 4));
   b.tok_pos = reinterpret_cast<int*>(take(M * 4));
+  b.qkv_split = (int)std::min<size_t>(GEMM_MAX_SPLIT, z.qkv / (M * nqkv * 4));
+  b.p_split = (int)std::max<size_t>(1, std::min<size_t>(GEMM_MAX_SPLIT, (z.qkv + M * hq * 4) / (M * c.d_model * 4)));
   return b;
 }
 
@@ -196,7 +210,6 @@ struct sk_engine {
   // batched prefill activations, sized for the largest packed prefix so far
   int pf_cap = 0;
   void* pf_mem = nullptr;
-  PrefillBufs pf;
   int* p_row_start = nullptr;
   float2* p_rope = nullptr;   // [max_ctx + 1][hd/2] (cos, sin) by position, filled at creation
 };
@@ -867,25 +880,32 @@ hipError_t enqueue_tail(sk_engine* e) {
 
 // Code tables of the depth steps (depth_step_kernel): P_j = (table[j] * norm_in
 // gain) W_gu^T for j < Q-1, [V][gate | up] per codebook, on the FP32 matrix
-// cores (BF16 weights widened exactly); derived from the weights bound when the
-// frame is captured.
+// cores (BF16 weights widened exactly first); derived from the weights bound
+// when the frame is captured.
 template <typename TL>
-hipError_t build_code_tables_t(sk_engine* e, float* tmp) {
+hipError_t build_code_tables_t(sk_engine* e, float* tmp, float* wide) {
   const sk_config& c = e->c;
   const int d = c.d_model, KI = c.depth_inner, V = c.audio_vocab;
   const size_t tsz = sizeof(typename TL::elem);
+  const void *gate = e->d_gate, *up = e->d_up;
+  if (tsz == 2) {
+    float* g32 = wide;
+    float* u32 = wide + (size_t)KI * d;
+    hipLaunchKernelGGL(scale_rows_kernel<TL>, dim3(1024), dim3(256), 0, e->stream, gate, (const float*)nullptr, KI, d, g32);
+    hipLaunchKernelGGL(scale_rows_kernel<TL>, dim3(1024), dim3(256), 0, e->stream, up, (const float*)nullptr, KI, d, u32);
+    gate = g32;
+    up = u32;
+  }
   for (int j = 0; j + 1 < c.n_codebooks; ++j) {
     const void* tj = static_cast<const char*>(e->table) + (size_t)j * V * d * tsz;
     hipLaunchKernelGGL(scale_rows_kernel<TL>, dim3(1024), dim3(256), 0, e->stream, tj, e->d_norm_in, V, d, tmp);
     GemmArgs g{};
-    g.A = tmp; g.lda = d;
-    g.B[0] = e->d_gate; g.B[1] = e->d_up; g.B[2] = nullptr;
-    g.seg_rows[0] = KI; g.seg_rows[1] = KI; g.seg_rows[2] = 0;
+    g.A = tmp;
+    g.B[0] = gate; g.B[1] = up;
+    g.seg_rows[0] = KI; g.seg_rows[1] = KI;
     g.out = e->ptab + (size_t)j * V * 2 * KI; g.ldo = 2 * KI;
-    g.M = V; g.N = 2 * KI; g.K = d;
-    hipLaunchKernelGGL((gemm_nt_kernel<GEPI_STORE, TL, 64>), dim3((2 * KI + GBN - 1) / GBN, (V + 63) / 64), dim3(256),
-                       0, e->stream, g);
-    const hipError_t err = hipGetLastError();
+    g.M = V; g.N = 2 * KI; g.K = d; g.ksplit = 1;
+    const hipError_t err = launch_gemm<GEPI_STORE>(false, 0, g, e->stream);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
@@ -898,10 +918,10 @@ int build_code_tables(sk_engine* e) {
     SK_HIP(dalloc(&e->gbuf[0], (size_t)e->rows * 2 * KI));
     SK_HIP(dalloc(&e->gbuf[1], (size_t)e->rows * 2 * KI));
   }
-  float* tmp = nullptr;
-  SK_HIP(dalloc(&tmp, V * d));
-  const hipError_t err = c.weight_dtype == SK_BF16 ? build_code_tables_t<WBF16>(e, tmp)
-                                                   : build_code_tables_t<WF32>(e, tmp);
+  const bool bf = c.weight_dtype == SK_BF16;
+  float* tmp = nullptr;   // a codebook's scaled table, then the widened gate and up weights
+  SK_HIP(dalloc(&tmp, V * d + (bf ? 2 * KI * d : 0)));
+  const hipError_t err = bf ? build_code_tables_t<WBF16>(e, tmp, tmp + V * d) : build_code_tables_t<WF32>(e, tmp, nullptr);
   const hipError_t serr = hipStreamSynchronize(e->stream);
   hipFree(tmp);
   SK_HIP(err);
@@ -911,105 +931,102 @@ int build_code_tables(sk_engine* e) {
 
 // ---- batched prefill -------------------------------------------------------
 
-// 64-row tiles unless they leave more than half the CUs idle, then 32-row tiles.
-template <int EPI>
-hipError_t launch_gemm(int wdtype, const GemmArgs& g, hipStream_t st) {
-  const int nt = (g.N + GBN - 1) / GBN;
-  const bool small = nt * ((g.M + 63) / 64) < 128;
-  const dim3 grid(nt, small ? (g.M + 31) / 32 : (g.M + 63) / 64);
-  if (wdtype == SK_BF16) {
-    if (small) hipLaunchKernelGGL((gemm_bf16_kernel<EPI, 32>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((gemm_bf16_kernel<EPI, 64>), grid, dim3(256), 0, st, g);
-  } else {   // FP32 weights stay on the FP32 matrix cores: exact FP32 products
-    if (small) hipLaunchKernelGGL((gemm_nt_kernel<EPI, WF32, 32>), grid, dim3(256), 0, st, g);
-    else hipLaunchKernelGGL((gemm_nt_kernel<EPI, WF32, 64>), grid, dim3(256), 0, st, g);
-  }
-  return hipGetLastError();
-}
-
-GemmArgs gemm_args(const float* A, int lda, const void* B, int M, int N, int K, float* out, int ldo) {
-  GemmArgs g{};
-  g.A = A; g.lda = lda;
-  g.B[0] = B; g.B[1] = nullptr; g.B[2] = nullptr;
-  g.seg_rows[0] = N; g.seg_rows[1] = 0; g.seg_rows[2] = 0;
-  g.out = out; g.ldo = ldo;
-  g.M = M; g.N = N; g.K = K;
-  return g;
-}
-
 hipError_t ensure_prefill_bufs(sk_engine* e, int M) {
   if (M <= e->pf_cap) return hipSuccess;
   if (e->pf_mem) hipFree(e->pf_mem);
   e->pf_mem = nullptr;
-  e->pf = PrefillBufs{};
   e->pf_cap = 0;
-  const hipError_t err = hipMalloc(&e->pf_mem, prefill_bytes(e->c, e->nqkv, M));
+  const hipError_t err = hipMalloc(&e->pf_mem, prefill_sizes(e->c, e->nqkv, M).total);
   if (err != hipSuccess) return err;
-  e->pf = carve_prefill(e->c, e->nqkv, M, e->pf_mem);
   e->pf_cap = M;
   return hipSuccess;
 }
 
-// All staged prefix tokens through the trunk at once (M = total tokens).
-hipError_t enqueue_batched_prefill(sk_engine* e, int M, int max_len, const PrefillBufs& b) {
+template <bool BF, int NCH>
+hipError_t launch_pf_norm_t(const sk_engine* e, bool first, int M, const PrefillBufs& b, int ns, size_t slice,
+                            const float* w) {
   const sk_config& c = e->c;
-  const int d = c.d_model, hd = c.head_dim, wt = c.weight_dtype;
-  const int hq = c.n_q_heads * hd, I = c.trunk_inter;
-  const bool bf = c.kv_dtype == SK_BF16;
+  hipLaunchKernelGGL((pf_norm_kernel<BF, NCH>), dim3(M), dim3(NT), 0, e->stream, first ? e->embeds : nullptr,
+                     c.max_ctx, b.tok_row, b.tok_pos, b.QKV, ns, slice, w, c.trunk_eps, c.d_model, b.X, b.Xn,
+                     reinterpret_cast<uint16_t*>(b.Xn), (size_t)M * c.d_model);
+  return hipGetLastError();
+}
+template <bool BF>
+hipError_t launch_pf_norm(const sk_engine* e, bool first, int M, const PrefillBufs& b, int ns, size_t slice,
+                          const float* w) {
+  const int d = e->c.d_model;
+  if (d <= 4 * NT) return launch_pf_norm_t<BF, 1>(e, first, M, b, ns, slice, w);
+  if (d <= 8 * NT) return launch_pf_norm_t<BF, 2>(e, first, M, b, ns, slice, w);
+  if (d <= 16 * NT) return launch_pf_norm_t<BF, 4>(e, first, M, b, ns, slice, w);
+  return launch_pf_norm_t<BF, 0>(e, first, M, b, ns, slice, w);
+}
+
+// KT: KV cache element; BF: BF16 weights (activations as hi and lo planes).
+template <typename KT, bool BF>
+hipError_t enqueue_prefill_t(sk_engine* e, int M, int max_len, const PrefillBufs& b) {
+  const sk_config& c = e->c;
+  const int d = c.d_model, hd = c.head_dim, hq = c.n_q_heads * hd, I = c.trunk_inter;
   hipStream_t st = e->stream;
   hipError_t err;
-  hipLaunchKernelGGL(pf_gather_kernel, dim3(M), dim3(NT), 0, st, e->embeds, c.max_ctx, b.tok_row,
-                     b.tok_pos, d, b.X);
-  if ((err = hipGetLastError()) != hipSuccess) return err;
   const size_t asmem = pf_attn_smem_floats(hd) * sizeof(float);
   const int G = c.n_q_heads / c.n_kv_heads, QB = PF_NQ / G;
+  const GemmPlan pq = plan_gemm(BF, false, M, e->nqkv, d, b.qkv_split), po = plan_gemm(BF, false, M, d, hq, b.p_split),
+                 pg = plan_gemm(BF, true, M, I, d, 1), pd = plan_gemm(BF, false, M, d, I, b.p_split);
+  // The O and down projections add to X themselves, or leave K slices in P for
+  // the next norm to add.
+  const size_t pslice = (size_t)M * d;
+  const int no = po.ksplit > 1 ? po.ksplit : 0, nd = pd.ksplit > 1 ? pd.ksplit : 0;
+  auto gemm = [&](const GemmPlan& p, const void* A, const void* B, int N, int K, float* out) {
+    GemmArgs g{};
+    g.A = A; g.a_lo = (size_t)M * K;
+    g.B[0] = B; g.seg_rows[0] = N;
+    g.out = out; g.ldo = N; g.slice = (size_t)M * N;
+    g.M = M; g.N = N; g.K = K; g.ksplit = p.ksplit;
+    return g;
+  };
   for (int l = 0; l < c.n_layers; ++l) {
     const LayerW& w = e->L[l];
-    char* kc = e->kc + (size_t)l * kv_layer_bytes(e);
-    char* vc = e->vc + (size_t)l * kv_layer_bytes(e);
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(M), dim3(NT), 0, st, b.X, (const float*)nullptr, w.in_norm,
-                       c.trunk_eps, d, b.Xn, (const int*)nullptr);
-    GemmArgs g = gemm_args(b.Xn, d, w.q, M, e->nqkv, d, b.QKV, e->nqkv);
+    KT* kc = reinterpret_cast<KT*>(e->kc + (size_t)l * kv_layer_bytes(e));
+    KT* vc = reinterpret_cast<KT*>(e->vc + (size_t)l * kv_layer_bytes(e));
+    if ((err = launch_pf_norm<BF>(e, l == 0, M, b, l == 0 ? 0 : nd, pslice, w.in_norm)) != hipSuccess) return err;
+    GemmArgs g = gemm(pq, b.Xn, w.q, e->nqkv, d, b.QKV);
     g.B[1] = w.k; g.B[2] = w.v;
     g.seg_rows[0] = hq; g.seg_rows[1] = c.n_kv_heads * hd; g.seg_rows[2] = c.n_kv_heads * hd;
-    if ((err = launch_gemm<GEPI_STORE>(wt, g, st)) != hipSuccess) return err;
-    if (bf)
-      hipLaunchKernelGGL(pf_qkv_kernel<uint16_t>, dim3(M), dim3(NT), 0, st, b.QKV, e->nqkv, b.tok_row,
-                         b.tok_pos, w.q_norm, w.k_norm, c.trunk_eps, e->p_rope, c.n_q_heads, c.n_kv_heads, hd,
-                         c.max_ctx, b.Q, reinterpret_cast<uint16_t*>(kc), reinterpret_cast<uint16_t*>(vc));
-    else
-      hipLaunchKernelGGL(pf_qkv_kernel<float>, dim3(M), dim3(NT), 0, st, b.QKV, e->nqkv, b.tok_row,
-                         b.tok_pos, w.q_norm, w.k_norm, c.trunk_eps, e->p_rope, c.n_q_heads, c.n_kv_heads, hd,
-                         c.max_ctx, b.Q, reinterpret_cast<float*>(kc), reinterpret_cast<float*>(vc));
+    if ((err = launch_gemm<GEPI_STORE>(BF, pq.tile, g, st)) != hipSuccess) return err;
+    hipLaunchKernelGGL(pf_qkv_kernel<KT>, dim3(M), dim3(NT), 0, st, b.QKV, e->nqkv, pq.ksplit, g.slice, b.tok_row,
+                       b.tok_pos, w.q_norm, w.k_norm, c.trunk_eps, e->p_rope, c.n_q_heads, c.n_kv_heads, hd,
+                       c.max_ctx, b.Q, kc, vc);
     const dim3 agrid((max_len + QB - 1) / QB, c.n_kv_heads, e->rows);
-    const float scale = 1.0f / sqrtf((float)hd);
-    if (bf)
-      hipLaunchKernelGGL(pf_attention_kernel<uint16_t>, agrid, dim3(NT), asmem, st, b.Q,
-                         reinterpret_cast<const uint16_t*>(kc), reinterpret_cast<const uint16_t*>(vc),
-                         e->p_row_start, e->plen, c.n_q_heads, c.n_kv_heads, hd, c.max_ctx, scale, b.ATT, hq);
-    else
-      hipLaunchKernelGGL(pf_attention_kernel<float>, agrid, dim3(NT), asmem, st, b.Q,
-                         reinterpret_cast<const float*>(kc), reinterpret_cast<const float*>(vc), e->p_row_start,
-                         e->plen, c.n_q_heads, c.n_kv_heads, hd, c.max_ctx, scale, b.ATT, hq);
+    hipLaunchKernelGGL((pf_attention_kernel<KT, BF>), agrid, dim3(NT), asmem, st, b.Q, kc, vc, e->p_row_start, e->plen,
+                       c.n_q_heads, c.n_kv_heads, hd, c.max_ctx, 1.0f / sqrtf((float)hd), b.ATT, hq,
+                       reinterpret_cast<uint16_t*>(b.ATT), (size_t)M * hq);
     if ((err = hipGetLastError()) != hipSuccess) return err;
-    g = gemm_args(b.ATT, hq, w.o, M, d, hq, b.X, d);
-    g.res = b.X; g.ldr = d;
-    if ((err = launch_gemm<GEPI_RESID>(wt, g, st)) != hipSuccess) return err;
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(M), dim3(NT), 0, st, b.X, (const float*)nullptr, w.post_norm,
-                       c.trunk_eps, d, b.Xn, (const int*)nullptr);
-    g = gemm_args(b.Xn, d, w.gate, M, I, d, b.ACT, I);
+    g = gemm(po, b.ATT, w.o, d, hq, no ? b.QKV : b.X);
+    g.res = no ? nullptr : b.X;
+    if ((err = launch_gemm<GEPI_STORE>(BF, po.tile, g, st)) != hipSuccess) return err;
+    if ((err = launch_pf_norm<BF>(e, false, M, b, no, pslice, w.post_norm)) != hipSuccess) return err;
+    g = gemm(pg, b.Xn, w.gate, I, d, b.ACT);
     g.B2 = w.up;
-    if ((err = launch_gemm<GEPI_SWIGLU>(wt, g, st)) != hipSuccess) return err;
-    g = gemm_args(b.ACT, I, w.down, M, d, I, b.X, d);
-    g.res = b.X; g.ldr = d;
-    if ((err = launch_gemm<GEPI_RESID>(wt, g, st)) != hipSuccess) return err;
+    g.xs = reinterpret_cast<uint16_t*>(b.ACT); g.xs_lo = (size_t)M * I;
+    if ((err = launch_gemm<GEPI_SWIGLU>(BF, pg.tile, g, st)) != hipSuccess) return err;
+    g = gemm(pd, b.ACT, w.down, d, I, nd ? b.QKV : b.X);
+    g.res = nd ? nullptr : b.X;
+    if ((err = launch_gemm<GEPI_STORE>(BF, pd.tile, g, st)) != hipSuccess) return err;
   }
-  hipLaunchKernelGGL(pf_finish_kernel, dim3(e->rows), dim3(NT), 0, st, b.X, e->p_row_start, e->plen,
-                     e->final_norm, c.trunk_eps, d, e->hidden, e->kv_len, e->pos, e->active, e->inv_freq, hd / 2,
-                     e->rope, e->d_norm_in, c.depth_eps, e->abuf, e->xs_abuf);
+  hipLaunchKernelGGL(pf_finish_kernel, dim3(e->rows), dim3(NT), 0, st, b.X, b.QKV, nd, pslice, e->p_row_start,
+                     e->plen, e->final_norm, c.trunk_eps, d, e->hidden, e->kv_len, e->pos, e->active, e->inv_freq,
+                     hd / 2, e->rope, e->d_norm_in, c.depth_eps, e->abuf, e->xs_abuf);
   const hipError_t fe = hipGetLastError();
   if (fe != hipSuccess || !e->code_tables) return fe;
   return launch_g1(e);
+}
+
+// All staged prefix tokens through the trunk at once (M = total tokens).
+hipError_t enqueue_batched_prefill(sk_engine* e, int M, int max_len, const PrefillBufs& b) {
+  const bool kb = e->c.kv_dtype == SK_BF16;
+  if (e->c.weight_dtype == SK_BF16)
+    return kb ? enqueue_prefill_t<uint16_t, true>(e, M, max_len, b) : enqueue_prefill_t<float, true>(e, M, max_len, b);
+  return kb ? enqueue_prefill_t<uint16_t, false>(e, M, max_len, b) : enqueue_prefill_t<float, false>(e, M, max_len, b);
 }
 
 int capture(sk_engine* e, hipError_t (*body)(sk_engine*), hipGraph_t* g, hipGraphExec_t* x) {
@@ -1445,7 +1462,7 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
   }
   PrefillBufs bufs;
   if (noalloc) {
-    const size_t need = prefill_bytes(e->c, e->nqkv, M);
+    const size_t need = prefill_sizes(e->c, e->nqkv, M).total;
     SK_CHECK(need <= SK_NOALLOC_SCRATCH_BYTES, SK_EINVAL,
              "prefill of %d packed tokens needs %zu bytes of scratch, more than the %zu of "
              "sk_prefill_run_noalloc (use sk_prefill_run)", M, need, (size_t)SK_NOALLOC_SCRATCH_BYTES);
@@ -1455,7 +1472,7 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
   } else {
     const hipError_t ae = ensure_prefill_bufs(e, M);
     SK_CHECK(ae == hipSuccess, SK_EHIP, "prefill buffers for %d tokens: %s", M, hipGetErrorString(ae));
-    bufs = e->pf;
+    bufs = carve_prefill(e->c, e->nqkv, M, e->pf_mem);
   }
   {
     // in the device's order of engines, like frames: no other engine's frame

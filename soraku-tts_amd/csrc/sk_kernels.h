@@ -2981,7 +2981,7 @@ template <typename TL>
 __global__ void scale_rows_kernel(const void* table, const float* gain, int rows, int d, float* out) {
   const size_t n = (size_t)rows * d;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    out[i] = TL::get(table, i) * gain[i % d];
+    out[i] = gain ? TL::get(table, i) * gain[i % d] : TL::get(table, i);   // null gain: widen only
 }
 
 // Standalone sampler (operator API): one utterance, parameters by value.
