@@ -961,6 +961,41 @@ hipError_t launch_pf_norm(const sk_engine* e, bool first, int M, const PrefillBu
   return launch_pf_norm_t<BF, 0>(e, first, M, b, ns, slice, w);
 }
 
+template <typename KT, int HD, int WK, bool BF>
+hipError_t launch_pf_attention_t(const sk_engine* e, int M, int max_len, const PrefillBufs& b, const KT* kc,
+                                 const KT* vc) {
+  const sk_config& c = e->c;
+  const int QB = PF_NQ / e->G, hq = c.n_q_heads * HD;
+  constexpr size_t smem = pf_attn_smem<KT, HD>(WK);
+  auto fn = pf_attention_kernel<KT, HD, WK, BF>;
+  if constexpr (smem > 65536) {
+    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (err != hipSuccess) return err;
+  }
+  hipLaunchKernelGGL(fn, dim3(c.n_kv_heads * e->rows, (max_len + QB - 1) / QB), dim3(WK * 64), smem, e->stream, b.Q,
+                     kc, vc, e->p_row_start, e->plen, c.n_q_heads, c.n_kv_heads, c.max_ctx, 1.0f / sqrtf((float)HD),
+                     b.ATT, hq, reinterpret_cast<uint16_t*>(b.ATT), (size_t)M * hq);
+  return hipGetLastError();
+}
+template <typename KT, bool BF>
+hipError_t launch_pf_attention(const sk_engine* e, int M, int max_len, const PrefillBufs& b, const KT* kc,
+                               const KT* vc) {
+  switch (e->c.head_dim) {
+    case 16: return launch_pf_attention_t<KT, 16, 4, BF>(e, M, max_len, b, kc, vc);
+    case 32: return launch_pf_attention_t<KT, 32, 4, BF>(e, M, max_len, b, kc, vc);
+    case 64: return launch_pf_attention_t<KT, 64, 4, BF>(e, M, max_len, b, kc, vc);
+    default: break;
+  }
+  // Keys cut 4 ways until the workgroups alone fill the GPU four deep, then 2
+  // ways (us per layer with 1 / 2 / 4 / 8: 1314 tokens, 660 workgroups 220 /
+  // 161 / 92 / 101; 241 + 146 tokens, 200 workgroups 46 / 27 / 17.5 / 17.7; 32
+  // rows of 60-240, 2350 workgroups 83 / 73 / 88 / 129).
+  const int QB = PF_NQ / e->G, wgs = (M + QB - 1) / QB * e->c.n_kv_heads;
+  return wgs < 1024 ? launch_pf_attention_t<KT, 128, 4, BF>(e, M, max_len, b, kc, vc)
+                    : launch_pf_attention_t<KT, 128, 2, BF>(e, M, max_len, b, kc, vc);
+}
+
 // KT: KV cache element; BF: BF16 weights (activations as hi and lo planes).
 template <typename KT, bool BF>
 hipError_t enqueue_prefill_t(sk_engine* e, int M, int max_len, const PrefillBufs& b) {
@@ -968,8 +1003,6 @@ hipError_t enqueue_prefill_t(sk_engine* e, int M, int max_len, const PrefillBufs
   const int d = c.d_model, hd = c.head_dim, hq = c.n_q_heads * hd, I = c.trunk_inter;
   hipStream_t st = e->stream;
   hipError_t err;
-  const size_t asmem = pf_attn_smem_floats(hd) * sizeof(float);
-  const int G = c.n_q_heads / c.n_kv_heads, QB = PF_NQ / G;
   const GemmPlan pq = plan_gemm(BF, false, M, e->nqkv, d, b.qkv_split), po = plan_gemm(BF, false, M, d, hq, b.p_split),
                  pg = plan_gemm(BF, true, M, I, d, 1), pd = plan_gemm(BF, false, M, d, I, b.p_split);
   // The O and down projections add to X themselves, or leave K slices in P for
@@ -996,11 +1029,8 @@ hipError_t enqueue_prefill_t(sk_engine* e, int M, int max_len, const PrefillBufs
     hipLaunchKernelGGL(pf_qkv_kernel<KT>, dim3(M), dim3(NT), 0, st, b.QKV, e->nqkv, pq.ksplit, g.slice, b.tok_row,
                        b.tok_pos, w.q_norm, w.k_norm, c.trunk_eps, e->p_rope, c.n_q_heads, c.n_kv_heads, hd,
                        c.max_ctx, b.Q, kc, vc);
-    const dim3 agrid((max_len + QB - 1) / QB, c.n_kv_heads, e->rows);
-    hipLaunchKernelGGL((pf_attention_kernel<KT, BF>), agrid, dim3(NT), asmem, st, b.Q, kc, vc, e->p_row_start, e->plen,
-                       c.n_q_heads, c.n_kv_heads, hd, c.max_ctx, 1.0f / sqrtf((float)hd), b.ATT, hq,
-                       reinterpret_cast<uint16_t*>(b.ATT), (size_t)M * hq);
     if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_pf_attention<KT, BF>(e, M, max_len, b, kc, vc)) != hipSuccess) return err;
     g = gemm(po, b.ATT, w.o, d, hq, no ? b.QKV : b.X);
     g.res = no ? nullptr : b.X;
     if ((err = launch_gemm<GEPI_STORE>(BF, po.tile, g, st)) != hipSuccess) return err;

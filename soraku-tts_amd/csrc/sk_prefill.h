@@ -13,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "sk_gemm.h"
 #include "sk_kernels.h"
 
@@ -164,198 +166,245 @@ __global__ __launch_bounds__(NT) void pf_qkv_kernel(const float* qkv, int ldqkv,
 }
 
 // ------------------------------------------------------------ causal attention
-// Grid (query blocks, Hkv, rows); the workgroup holds PF_NQ = 32 query
-// vectors: the G heads of kv head h for QB = 32 / G consecutive positions of
-// the row, and walks the row's keys 0 .. (last query position) in chunks of
-// 32 with an online softmax (scale hd^-1/2, keys after the query masked).
-// Per chunk: S = Q K^T on the matrix cores (one 16 x 16 tile per wave, Q
-// fragments kept in registers), softmax over each query's 32 scores by 8
-// threads (DPP all-reduce), O += P V on the matrix cores.  K / V come from
-// the cache just written (BF16 widened), so attention sees exactly what
-// decode steps will see.
-constexpr int PF_NQ = 32, PF_KC = 32;
+// The workgroup holds PF_NQ = 32 query vectors (two MFMA tiles of 16): the G
+// heads of kv head h for 32 / G consecutive positions of row r.  Its WK waves
+// share the keys up to the last query position, 16 at a time (wave w takes
+// tiles w, w + WK, ...), each with its own online softmax; the partial
+// outputs meet in LDS at the end.  No barrier and no LDS inside the loop:
+//   S^T = K Q^T on the FP32 matrix cores (v_mfma_f32_16x16x4f32): lane l holds
+//     the scores of query l % 16 for keys 4 (l / 16) + v, v < 4;
+//   the softmax of a query is 4 values per lane and two exchanges between
+//     lanes 16 and 32 apart;
+//   O^T += V^T P^T takes those four values as they are: step v multiplies the
+//     keys 4 q + v, q = 0 .. 3, of P (this lane's) and V (row 4 q + v).
+// K and V come straight from the cache just written (BF16 widened), 16 bytes
+// per lane, V of a tile in flight under S, the next K under the softmax and
+// PV.  A K load gives dims KW q + e of key l % 16 to lane l (q = l / 16), a V
+// load dims VW i + e of keys 4 q + v to lane i + 16 q; Q is loaded in K's
+// order, and O's rows come out in V's.
+//
+// What bounds it: FP32 MFMA time (40% of the kernel on long prefixes) with the
+// softmax, rescaling and merge arithmetic beside it; workgroups with the
+// longest walk start first.  Tried: K of the next tile loaded under a branch or
+// past the end of the keys (PV then waits for it, 29 -> 40 us on the pair
+// below).  us per layer before (32 queries per workgroup through LDS, four
+// barriers per 32 keys) -> now: 1314 tokens, 1.7B 224 -> 92; 241 + 146 tokens
+// 34 -> 17.5; 32 rows of 60-240 tokens, BF16 cache 133 -> 73.
+constexpr int PF_NQ = 32;
 
-__host__ __device__ constexpr int pf_ldk(int hd) { return hd + 2; }    // lanes 0-15: 16 rows, 2 banks apart
-__host__ __device__ constexpr int pf_ldv(int hd) { return hd + 16; }   // lanes 16-31: next row, 16 banks on
-constexpr int PF_LDS = PF_KC + 1;
-__host__ __device__ constexpr size_t pf_attn_smem_floats(int hd) {
-  return (size_t)PF_KC * pf_ldk(hd) + (size_t)PF_KC * pf_ldv(hd) + (size_t)PF_NQ * PF_LDS + 2 * (size_t)PF_NQ;
+template <typename KT, int HD>
+struct PfAttDims {
+  static constexpr int KW = (16 / (int)sizeof(KT)) < HD / 4 ? 16 / (int)sizeof(KT) : HD / 4;   // dims per K load
+  static constexpr int NK = HD / (4 * KW);                                                     // K loads per tile
+  static constexpr int NDT = HD / 16;                                                          // 16-dim output tiles
+  static constexpr int VW = (16 / (int)sizeof(KT)) < NDT ? 16 / (int)sizeof(KT) : NDT;         // dims per V load
+  static constexpr int NV = NDT / VW;                                                          // V loads per key row
+  static constexpr int LDO = HD + 4;                                                           // merge row stride
+};
+template <typename KT, int HD>
+constexpr size_t pf_attn_smem(int wk) {   // bytes: partial outputs, then (max, sum) per wave and query
+  return ((size_t)wk * PF_NQ * PfAttDims<KT, HD>::LDO + 2 * (size_t)wk * PF_NQ) * sizeof(float);
 }
 
-// all-reduce over each aligned group of 8 lanes
-__device__ __forceinline__ float grp8_max(float v) {
-  v = fmaxf(v, dpp_keep<0xb1, 0xf>(v));    // quad_perm [1,0,3,2]
-  v = fmaxf(v, dpp_keep<0x4e, 0xf>(v));    // quad_perm [2,3,0,1]
-  return fmaxf(v, dpp_keep<0x141, 0xf>(v));  // row_half_mirror: lane i <-> 7 - i
-}
-__device__ __forceinline__ float grp8_sum(float v) {
-  v += dpp_keep<0xb1, 0xf>(v);
-  v += dpp_keep<0x4e, 0xf>(v);
-  return v + dpp_keep<0x141, 0xf>(v);
-}
+// N consecutive cache elements as loaded; get<i>() widens one to FP32 (kept
+// packed until used: half the registers with BF16).
+template <typename KT, int N>
+struct KvPiece {
+  uint32_t w[(N * sizeof(KT) + 3) / 4];
+  __device__ __forceinline__ void load(const KT* base, unsigned off) {   // off in bytes
+    const char* p = reinterpret_cast<const char*>(base) + off;
+    if constexpr (N * sizeof(KT) == 16) {
+      const uint4 v = *reinterpret_cast<const uint4*>(p);
+      w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+    } else if constexpr (N * sizeof(KT) == 8) {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      w[0] = v.x; w[1] = v.y;
+    } else if constexpr (N * sizeof(KT) == 4) {
+      w[0] = *reinterpret_cast<const uint32_t*>(p);
+    } else {
+      w[0] = *reinterpret_cast<const uint16_t*>(p);
+    }
+  }
+  __device__ __forceinline__ float get(int i) const {
+    if constexpr (sizeof(KT) == 4) return __uint_as_float(w[i]);
+    else return __uint_as_float(i & 1 ? w[i / 2] & 0xffff0000u : w[i / 2] << 16);
+  }
+};
 
-template <typename KT, bool BF>
-__global__ __launch_bounds__(NT) void pf_attention_kernel(const float* Q, const KT* kc, const KT* vc,
-                                                          const int* row_start, const int* len, int Hq, int Hkv,
-                                                          int hd, int max_ctx, float scale, float* out, int ldo,
-                                                          uint16_t* xs, size_t xs_lo) {
+template <typename KT, int HD, int WK, bool BF>
+__global__ __launch_bounds__(WK * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void pf_attention_kernel(
+    const float* Q, const KT* kc, const KT* vc, const int* row_start, const int* len, int Hq, int Hkv, int max_ctx,
+    float scale, float* out, int ldo, uint16_t* xs, size_t xs_lo) {
+  using D = PfAttDims<KT, HD>;
+  constexpr int KW = D::KW, NK = D::NK, NDT = D::NDT, VW = D::VW, NV = D::NV, LDO = D::LDO;
   extern __shared__ __attribute__((aligned(16))) float psm[];
   const int G = Hq / Hkv, QB = PF_NQ / G;
-  const int qb = blockIdx.x, h = blockIdx.y, r = blockIdx.z;
-  const int n = len[r];
-  const int p0 = qb * QB;
+  const int h = blockIdx.x % Hkv, r = blockIdx.x / Hkv;
+  const int n = len[r], p0 = (int)(gridDim.y - 1 - blockIdx.y) * QB;
   if (p0 >= n) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ldk = pf_ldk(hd), ldv = pf_ldv(hd);
-  float* Ks = psm;                              // [KC][ldk]
-  float* Vs = Ks + PF_KC * ldk;                 // [KC][ldv]
-  float* P = Vs + PF_KC * ldv;                  // [NQ][PF_LDS] scores, then probabilities
-  float* Msc = P + PF_NQ * PF_LDS;              // [NQ] rescale of this chunk
-  float* Ml = Msc + PF_NQ;                      // [NQ] final sums
-  const size_t head_base = ((size_t)r * Hkv + h) * max_ctx;
-  const int m0 = row_start[r];
-  // query vector qv = g * QB + tq: head h * G + g at position p0 + tq
-  auto qpos = [&](int qv) { return p0 + (qv - (qv / QB) * QB); };
-  auto qhead = [&](int qv) { return h * G + qv / QB; };
-  const int i16 = lane & 15, k4 = lane >> 4;
-  // S tile of this wave: queries [16 qi, +16), keys [16 ki, +16)
-  const int qi = wave >> 1, ki = wave & 1;
-  float qf[32];                                 // A fragments over hd / 4 k-steps
-  {
-    const int qv = qi * 16 + i16;
-    const int p = min(qpos(qv), n - 1);
-    const float* qrow = Q + ((size_t)(m0 + p) * Hq + qhead(qv)) * hd;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i16 = lane & 15, q4 = lane >> 4;
+  const int m0 = row_start[r], last_p = min(p0 + QB, n) - 1;
+  const KT* kb = kc + ((size_t)r * Hkv + h) * max_ctx * HD;
+  const KT* vb = vc + ((size_t)r * Hkv + h) * max_ctx * HD;
+  // query vector qv = g * QB + t: head h * G + g at position p0 + t
+  int qp[2];
+  float qf[2][NK * KW];
 #pragma unroll
-    for (int ks = 0; ks < 32; ++ks) qf[ks] = (ks * 4 < hd) ? qrow[ks * 4 + k4] : 0.f;
-  }
-  // softmax role: query tid / 8, keys (tid % 8) * 4 .. + 4
-  const int sq = tid >> 3, sk0 = (tid & 7) * 4;
-  const int sp = qpos(sq);
-  float m_run = -INFINITY, l_run = 0.f;
-  // PV tiles of this wave: (query tile, d tile) pairs t = wave, wave + 4, ...
-  const int ndt = hd / 16, ntile = 2 * ndt;
-  v4f o[4];
+  for (int j = 0; j < 2; ++j) {
+    const int qv = j * 16 + i16, g = qv / QB;
+    qp[j] = p0 + qv - g * QB;
+    const float* qr = Q + ((size_t)(m0 + min(qp[j], n - 1)) * Hq + h * G + g) * HD;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
-  const int last_p = min(p0 + QB, n) - 1;
-  // K / V chunk staging: groups of 4 dims, up to 4 per thread (hd <= 128),
-  // loaded one chunk ahead into registers.
-  const int q4 = hd / 4, n4 = PF_KC * q4;
-  float4 kr[4], vr[4];
-  auto fetch = [&](int k0) {
+    for (int t = 0; t < NK; ++t)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = min(tid + u * NT, n4 - 1);
-      const int j = i / q4, d = (i - j * q4) * 4;
-      const size_t off = (head_base + min(k0 + j, n - 1)) * hd + d;
-      if constexpr (sizeof(KT) == 2) {
-        const uint2 kb = *reinterpret_cast<const uint2*>(kc + off);
-        const uint2 vb = *reinterpret_cast<const uint2*>(vc + off);
-        kr[u] = make_float4(__uint_as_float(kb.x << 16), __uint_as_float(kb.x & 0xffff0000u),
-                            __uint_as_float(kb.y << 16), __uint_as_float(kb.y & 0xffff0000u));
-        vr[u] = make_float4(__uint_as_float(vb.x << 16), __uint_as_float(vb.x & 0xffff0000u),
-                            __uint_as_float(vb.y << 16), __uint_as_float(vb.y & 0xffff0000u));
-      } else {   // built element-wise like the BF16 form, which keeps kr / vr in registers
-        const float4 kb = *reinterpret_cast<const float4*>(kc + off);
-        const float4 vb = *reinterpret_cast<const float4*>(vc + off);
-        kr[u] = make_float4(kb.x, kb.y, kb.z, kb.w);
-        vr[u] = make_float4(vb.x, vb.y, vb.z, vb.w);
+      for (int e = 0; e < KW; e += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(qr + t * 4 * KW + KW * q4 + e);
+        qf[j][t * KW + e] = v.x; qf[j][t * KW + e + 1] = v.y; qf[j][t * KW + e + 2] = v.z; qf[j][t * KW + e + 3] = v.w;
       }
+  }
+  KvPiece<KT, KW> kf[NK];
+  KvPiece<KT, VW> vf[4][NV];
+  auto load_k = [&](int k0) {
+    const unsigned p = (unsigned)(min(k0 + i16, n - 1) * HD + KW * q4) * sizeof(KT);
+#pragma unroll
+    for (int t = 0; t < NK; ++t) kf[t].load(kb, p + t * 4 * KW * sizeof(KT));
+  };
+  auto load_v = [&](int k0) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const unsigned p = (unsigned)(min(k0 + 4 * q4 + v, n - 1) * HD + VW * i16) * sizeof(KT);
+#pragma unroll
+      for (int t = 0; t < NV; ++t) vf[v][t].load(vb, p + t * 16 * VW * sizeof(KT));
     }
   };
-  fetch(0);
-  for (int k0 = 0; k0 <= last_p; k0 += PF_KC) {
-    __syncthreads();
+  v4f o[2][NDT];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int i = tid + u * NT;
-      if (i < n4) {
-        const int j = i / q4, d = (i - j * q4) * 4;
-        float2* kd = reinterpret_cast<float2*>(Ks + j * ldk + d);
-        kd[0] = make_float2(kr[u].x, kr[u].y);
-        kd[1] = make_float2(kr[u].z, kr[u].w);
-        *reinterpret_cast<float4*>(Vs + j * ldv + d) = vr[u];
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int t = 0; t < NDT; ++t) o[j][t] = v4f{0.f, 0.f, 0.f, 0.f};
+  float mr[2] = {-INFINITY, -INFINITY}, lr[2] = {0.f, 0.f};
+  const int k_first = wave * 16;
+  // one tile; `next`: the K of the wave's next tile is loaded on the way (a
+  // template argument: with a branch the compiler would make PV wait for those
+  // loads too)
+  auto tile = [&](int k0, auto next) {
+    load_v(k0);
+    v4f s[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int t = 0; t < NK; ++t)
+#pragma unroll
+      for (int e = 0; e < KW; ++e) {
+        const float k = kf[t].get(e);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, qf[j][t * KW + e], s[j], 0, 0, 0);
       }
-    }
-    __syncthreads();
-    if (k0 + PF_KC <= last_p) fetch(k0 + PF_KC);
-    // S tile = Q K^T
-    {
-      v4f sacc = v4f{0.f, 0.f, 0.f, 0.f};
-      const float* kp = Ks + (ki * 16 + i16) * ldk + k4;
+    if constexpr (decltype(next)::value) load_k(k0 + WK * 16);
 #pragma unroll
-      for (int ks = 0; ks < 32; ++ks)
-        if (ks * 4 < hd) sacc = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[ks], kp[ks * 4], sacc, 0, 0, 0);
-      const int key = k0 + ki * 16 + i16;
+    for (int j = 0; j < 2; ++j) {
+      float mx = -INFINITY;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int qv = qi * 16 + 4 * k4 + v;
-        const int pq = qpos(qv);
-        const bool ok = key <= pq && pq < n;
-        P[qv * PF_LDS + ki * 16 + i16] = ok ? sacc[v] * scale : -INFINITY;
+        const int key = k0 + 4 * q4 + v;
+        s[j][v] = key <= qp[j] && key < n ? s[j][v] * scale : -INFINITY;
+        mx = fmaxf(mx, s[j][v]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(mr[j], mx);
+      const bool none = mn == -INFINITY;         // every key so far is masked for this query
+      const float sc = none ? 1.f : expf(mr[j] - mn);
+      float sum = 0.f;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        s[j][v] = none ? 0.f : expf(s[j][v] - mn);
+        sum += s[j][v];
+      }
+      lr[j] = lr[j] * sc + sum;                  // this lane's keys; the four lanes of a query add up at the end
+      mr[j] = mn;
+      if (__any(sc != 1.f)) {                    // some query's maximum moved
+#pragma unroll
+        for (int t = 0; t < NDT; ++t) o[j][t] *= sc;
       }
     }
-    __syncthreads();
-    // online softmax of query sq over its 32 scores (8 threads, 4 each)
-    {
-      float sv[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sv[j] = P[sq * PF_LDS + sk0 + j];
-      const float mx = grp8_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])));
-      const float mn = fmaxf(m_run, mx);
-      const bool none = (mn == -INFINITY);
-      const float sc = none ? 1.f : expf(m_run - mn);
-      float part = 0.f;
+    for (int v = 0; v < 4; ++v)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float e = none ? 0.f : expf(sv[j] - mn);
-        P[sq * PF_LDS + sk0 + j] = e;
-        part += e;
-      }
-      l_run = l_run * sc + grp8_sum(part);
-      m_run = mn;
-      if ((tid & 7) == 0) Msc[sq] = sc;
-    }
-    __syncthreads();
-    // O = O * rescale + P V
+      for (int t = 0; t < NV; ++t)
 #pragma unroll
-    for (int t4 = 0; t4 < 4; ++t4) {
-      const int t = wave + 4 * t4;
-      if (t < ntile) {
-        const int tq = t / ndt, td = t - tq * ndt;
+        for (int e = 0; e < VW; ++e) {
+          const float x = vf[v][t].get(e);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) o[t4][v] *= Msc[tq * 16 + 4 * k4 + v];
-        const float* pp = P + (tq * 16 + i16) * PF_LDS + k4;
-        const float* vp = Vs + k4 * ldv + td * 16 + i16;
-#pragma unroll
-        for (int ks = 0; ks < PF_KC / 4; ++ks)
-          o[t4] = __builtin_amdgcn_mfma_f32_16x16x4f32(pp[ks * 4], vp[ks * 4 * ldv], o[t4], 0, 0, 0);
-      }
-    }
+          for (int j = 0; j < 2; ++j)
+            o[j][t * VW + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, s[j][v], o[j][t * VW + e], 0, 0, 0);
+        }
+  };
+  if (k_first <= last_p) {
+    load_k(k_first);
+    int k0 = k_first;
+    for (; k0 + WK * 16 <= last_p; k0 += WK * 16) tile(k0, std::true_type{});
+    tile(k0, std::false_type{});
   }
-  if ((tid & 7) == 0) Ml[sq] = l_run;
-  __syncthreads();
+  // merge: every wave's partial output rows and (max, sum) per query
+  float* po = psm;                               // [WK][NQ][LDO]
+  float* pm = psm + WK * PF_NQ * LDO;            // [WK][NQ] max, then [WK][NQ] sum
+  float* pl = pm + WK * PF_NQ;
 #pragma unroll
-  for (int t4 = 0; t4 < 4; ++t4) {
-    const int t = wave + 4 * t4;
-    if (t < ntile) {
-      const int tq = t / ndt, td = t - tq * ndt;
+  for (int j = 0; j < 2; ++j) {
+    float l = lr[j];
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (q4 == 0) { pm[wave * PF_NQ + j * 16 + i16] = mr[j]; pl[wave * PF_NQ + j * 16 + i16] = l; }
+    float* row = po + (size_t)(wave * PF_NQ + j * 16 + i16) * LDO;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int qv = tq * 16 + 4 * k4 + v;
-        const int pq = qpos(qv);
-        if (pq < n) {
-          const float y = o[t4][v] / Ml[qv];
-          const size_t at = (size_t)(m0 + pq) * ldo + (size_t)qhead(qv) * hd + td * 16 + i16;
-          if constexpr (BF) {   // the O projection's input: BF16 hi and lo planes
-            const __bf16 hi = (__bf16)y;
-            xs[at] = __builtin_bit_cast(uint16_t, hi);
-            xs[at + xs_lo] = __builtin_bit_cast(uint16_t, (__bf16)(y - (float)hi));
-          } else {
-            out[at] = y;
-          }
+    for (int t = 0; t < NV; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {              // rows 4 q + v of tile (t, e): dim 16 VW t + VW (4 q + v) + e
+        float* d = row + 16 * VW * t + VW * (4 * q4 + v);
+        if constexpr (VW % 4 == 0) {
+#pragma unroll
+          for (int e = 0; e < VW; e += 4)
+            *reinterpret_cast<float4*>(d + e) = make_float4(o[j][t * VW + e][v], o[j][t * VW + e + 1][v],
+                                                            o[j][t * VW + e + 2][v], o[j][t * VW + e + 3][v]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < VW; ++e) d[e] = o[j][t * VW + e][v];
         }
       }
+  }
+  __syncthreads();
+  if (tid < PF_NQ) {                             // each wave's factor for query tid, in place of its max
+    float mx = -INFINITY, l = 0.f, f[WK];
+#pragma unroll
+    for (int w = 0; w < WK; ++w) mx = fmaxf(mx, pm[w * PF_NQ + tid]);   // finite: key 0 is wave 0's
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      f[w] = expf(pm[w * PF_NQ + tid] - mx);
+      l = fmaf(f[w], pl[w * PF_NQ + tid], l);
+    }
+#pragma unroll
+    for (int w = 0; w < WK; ++w) pm[w * PF_NQ + tid] = f[w] / l;
+  }
+  __syncthreads();
+  constexpr int NF = HD / 4;                     // float4 per output row
+  for (int it = tid; it < PF_NQ * NF; it += WK * 64) {
+    const int qv = it / NF, d = (it - qv * NF) * 4, g = qv / QB, pos = p0 + qv - g * QB;
+    if (pos >= n) continue;
+    float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      const float wt = pm[w * PF_NQ + qv];
+      const float4 x = *reinterpret_cast<const float4*>(po + (size_t)(w * PF_NQ + qv) * LDO + d);
+      y.x = fmaf(wt, x.x, y.x); y.y = fmaf(wt, x.y, y.y); y.z = fmaf(wt, x.z, y.z); y.w = fmaf(wt, x.w, y.w);
+    }
+    const size_t at = (size_t)(m0 + pos) * ldo + (size_t)(h * G + g) * HD + d;
+    if constexpr (BF) {                          // the O projection's input: BF16 hi and lo planes
+      uint2 hi, lo;
+      split4(y, hi, lo);
+      *reinterpret_cast<uint2*>(xs + at) = hi;
+      *reinterpret_cast<uint2*>(xs + at + xs_lo) = lo;
+    } else {
+      *reinterpret_cast<float4*>(out + at) = y;
     }
   }
 }
