@@ -124,7 +124,7 @@ struct sk_engine {
   int rows = 0, G = 0, nqkv = 0, inner_max = 0, max_chunks = 0;
   bool wide = false;          // more rows than the GEMV kernels take: skinny MFMA GEMMs
   int attn_splits = 0;        // > 0: attention_stream_kernel with this many splits per (row, kv head)
-  bool split_k = false;       // many-row BF16 GEMMs may split K (workgroups i, i + 8, ... share an XCD)
+  bool split_k = false;       // many-row GEMMs may split K (workgroups i, i + 8, ... share an XCD)
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t order_ev = nullptr;   // recorded on `stream` when another engine's frames follow this one's
@@ -387,38 +387,6 @@ int check_decode_weights(const sk_engine* e) {
 
 // ---- many-row path: skinny MFMA GEMMs ---------------------------------------
 
-// 16 waves per workgroup (K split 16 ways) when there are few workgroups
-// (N <= 1024 outputs, one weight matrix), else 8.  NORM: RMSNorm of x folded in.
-template <int EPI, bool NORM, typename WL>
-hipError_t launch_skinny_w(const SkinnyArgs& a, hipStream_t st) {
-  const dim3 grid((a.N + 15) / 16);
-  if (EPI != EPI_SWIGLU && a.N <= 1024)
-    hipLaunchKernelGGL((skinny_gemm_kernel<EPI, WL, 16, NORM>), grid, dim3(16 * 64), 0, st, a);
-  else
-    hipLaunchKernelGGL((skinny_gemm_kernel<EPI, WL, 8, NORM>), grid, dim3(8 * 64), 0, st, a);
-  return hipGetLastError();
-}
-// BF16 weights: K split over 4 or 2 workgroups per output tile when the
-// tiles alone would fill fewer than 256 CUs (tiles a multiple of 8, K slices
-// a multiple of 32); the slice partials live in `partial`, the arrival counts
-// in `arrive` (zero between launches).
-template <int EPI, bool NORM>
-hipError_t launch_skinny_bf16(SkinnyArgs a, float* partial, unsigned* arrive, bool allow_split, hipStream_t st) {
-  const int tiles = (a.N + 15) / 16;
-  a.ksplit = 1;
-  if (allow_split && tiles % 8 == 0) {
-    if (tiles <= 64 && a.K % (4 * 32) == 0) a.ksplit = 4;
-    else if (tiles <= 128 && a.K % (2 * 32) == 0) a.ksplit = 2;
-  }
-  static_assert(SK_MAX_SPLIT >= 4, "the kernel's split-K merge covers the splits chosen here");
-  a.partial = partial; a.arrive = arrive;
-  const dim3 grid(tiles * a.ksplit);
-  if (a.xs)
-    hipLaunchKernelGGL((skinny_bf16_kernel<EPI, 8, NORM, true>), grid, dim3(8 * 64), 0, st, a);
-  else
-    hipLaunchKernelGGL((skinny_bf16_kernel<EPI, 8, NORM, false>), grid, dim3(8 * 64), 0, st, a);
-  return hipGetLastError();
-}
 template <int EPI, bool NORM = false>
 hipError_t launch_skinny(sk_engine* e, const SkinnyArgs& a0) {
   SkinnyArgs a = a0;
@@ -426,18 +394,9 @@ hipError_t launch_skinny(sk_engine* e, const SkinnyArgs& a0) {
     a.tpart = e->sk_tpart; a.fc = e->fc; a.tag_idx = e->sk_tags++;
     a.err = e->sk_err; a.spin = e->spin_ticks;
   }
-  return e->c.weight_dtype == SK_BF16 ? launch_skinny_bf16<EPI, NORM>(a, e->sk_partial, e->sk_arrive, e->split_k,
-                                                                      e->stream)
-                                      : launch_skinny_w<EPI, NORM, WF32>(a, e->stream);
-}
-
-SkinnyArgs skinny_args(const void* w, int N, int K, const float* x, int ldx, float* out, int ldo, int R) {
-  SkinnyArgs a{};
-  a.w[0] = w; a.w[1] = nullptr; a.w[2] = nullptr;
-  a.seg_rows[0] = N; a.seg_rows[1] = 0; a.seg_rows[2] = 0;
-  a.x = x; a.ldx = ldx; a.out = out; a.ldo = ldo;
-  a.R = R; a.N = N; a.K = K;
-  return a;
+  a.partial = e->sk_partial;
+  a.arrive = e->sk_arrive;
+  return launch_skinny_w<EPI, NORM>(e->c.weight_dtype == SK_BF16, a, e->split_k, e->stream);
 }
 
 // Chunked decode attention: one workgroup per 32-token chunk of each (row,
@@ -1297,7 +1256,7 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
     if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
   }
   if (he == hipSuccess) he = prepare_sampler();
-  if (he == hipSuccess && e->wide && c.weight_dtype == SK_BF16) he = probe_xcd_mapping(e->stream, &e->split_k);
+  if (he == hipSuccess && e->wide) he = probe_xcd_mapping(e->stream, &e->split_k);
   // XCD-resident layers: the shape fits, the device has 8 x 32 CUs, workgroups
   // whose ids agree mod 8 share an XCD, and SORAKU_XCD_LAYERS is not "0"
   if (he == hipSuccess && lx_fits(e)) {

@@ -9,6 +9,7 @@
 #include "sk_error.h"
 #include "sk_kernels.h"
 #include "sk_launch.h"
+#include "sk_wide.h"
 #include "soraku_mi355x.h"
 
 using namespace sk;
@@ -22,16 +23,27 @@ int check_wdtype(int32_t wdtype) {
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Runs a GEMV over B activation rows in chunks of at most 4 rows.
-template <int PRO, int EPI>
-int gemv_rows(hipStream_t st, int wdtype, int B, GemvArgs a, int ldres) {
-  for (int b0 = 0; b0 < B; b0 += 4) {
-    const int m = (B - b0) < 4 ? (B - b0) : 4;
-    GemvArgs c = a;
-    c.x = a.x + (size_t)b0 * a.ldx;
-    c.out = a.out + (size_t)b0 * a.ldo;
-    if (a.res) c.res = a.res + (size_t)b0 * ldres;
-    SK_HIP((launch_gemv<PRO, EPI>(wdtype, m, c, st)));
+// A projection of B activation rows.  Up to 4 rows: the GEMV kernels.  More:
+// 32 rows per launch on the FP32 matrix cores (skinny_kernel), where one pass
+// over the weights serves them all (in chunks of 4 rows through the GEMV the
+// weights were read B / 4 times).  us per call, GEMV chunks / one pass: 4 rows,
+// FP32 2051 x 1024 5.2 / 5.6, BF16 2 x 2688 x 1344 8.7 / 11.5; 7 rows 8.5 / 5.6
+// and 14.7 / 11.7, BF16 2 x 6144 x 2048 34 / 18, 2048 x 6144 36 / 15; 20 rows,
+// FP32 2051 x 1024 20 / 7.4.
+constexpr int ROWS_GEMV = 4;
+template <int EPI>
+int project_rows(hipStream_t st, int wdtype, int B, const GemvArgs& a) {
+  if (B <= ROWS_GEMV) {
+    SK_HIP((launch_gemv<PRO_NONE, EPI>(wdtype, B, a, st)));
+    return SK_OK;
+  }
+  for (int b0 = 0; b0 < B; b0 += SK_ROWS) {
+    SkinnyArgs k = skinny_args(a.w[0], a.N, a.K, a.x + (size_t)b0 * a.ldx, a.ldx, a.out + (size_t)b0 * a.ldo, a.ldo,
+                               B - b0 < SK_ROWS ? B - b0 : SK_ROWS);
+    k.w2 = a.w[1];
+    k.bias = a.bias;
+    if (a.res) { k.res = a.res + (size_t)b0 * a.ldr; k.ldr = a.ldr; }
+    SK_HIP((launch_rows<EPI>(wdtype == SK_BF16, k, st)));
   }
   return SK_OK;
 }
@@ -69,7 +81,7 @@ int sk_op_swiglu_gemv(void* stream, int32_t B, int32_t I, int32_t D, int32_t wdt
   SK_CHECK(aligned16(x) && aligned16(wg) && aligned16(wu), SK_EINVAL, "operands must be 16-byte aligned");
   GemvArgs a = gemv_args(wg, I, D, x, D, out, I);
   a.w[1] = wu;
-  return gemv_rows<PRO_NONE, EPI_SWIGLU>((hipStream_t)stream, wdtype, B, a, 0);
+  return project_rows<EPI_SWIGLU>((hipStream_t)stream, wdtype, B, a);
 }
 
 int sk_op_down_residual_gemv(void* stream, int32_t B, int32_t D, int32_t I, int32_t wdtype,
@@ -81,7 +93,7 @@ int sk_op_down_residual_gemv(void* stream, int32_t B, int32_t D, int32_t I, int3
   SK_CHECK(aligned16(act) && aligned16(wd), SK_EINVAL, "operands must be 16-byte aligned");
   GemvArgs a = gemv_args(wd, D, I, act, I, out, D);
   a.res = residual; a.ldr = D;
-  return gemv_rows<PRO_NONE, EPI_RESID>((hipStream_t)stream, wdtype, B, a, D);
+  return project_rows<EPI_RESID>((hipStream_t)stream, wdtype, B, a);
 }
 
 int sk_op_classifier_gemv(void* stream, int32_t B, int32_t V, int32_t D, int32_t wdtype,
@@ -93,7 +105,7 @@ int sk_op_classifier_gemv(void* stream, int32_t B, int32_t V, int32_t D, int32_t
   SK_CHECK(aligned16(body) && aligned16(wq), SK_EINVAL, "operands must be 16-byte aligned");
   GemvArgs a = gemv_args(wq, V, D, body, D, out, V);
   a.bias = bias;
-  return gemv_rows<PRO_NONE, EPI_BIAS>((hipStream_t)stream, wdtype, B, a, 0);
+  return project_rows<EPI_BIAS>((hipStream_t)stream, wdtype, B, a);
 }
 
 int sk_op_frame_embed(void* stream, int32_t R, int32_t Q, int32_t V, int32_t D, float scale,

@@ -2,8 +2,8 @@
 // utterances with CFG decoded together, up to 32 rows (the reference decodes
 // one utterance's two CFG rows; fast_generate.py:232-328 batches those).
 //
-// The projections run as skinny GEMMs on the FP32 matrix cores: each
-// workgroup owns 16 outputs for all rows and splits K over its 8 or 16 waves;
+// The projections run as skinny GEMMs on the matrix cores: each
+// workgroup owns 16 outputs for all rows and splits K over its waves;
 // the per-wave partial tiles are summed through LDS in fixed wave order
 // (deterministic).  RMSNorms that feed a projection are folded into it.
 #pragma once
@@ -15,6 +15,7 @@
 #include "sk_kernels.h"
 
 namespace sk {
+namespace {   // internal linkage, as sk_kernels.h: both translation units include these kernels
 
 struct SkinnyArgs {
   const void* w[3]; int seg_rows[3];   // weight segments (q / k / v), rows of each
@@ -25,10 +26,10 @@ struct SkinnyArgs {
   const float* res; int ldr;           // residual (may alias out)
   const float* bias;                   // [N]
   int R, N, K;
-  int ksplit;                          // K slices per output tile (1, 2 or 4; BF16 form)
+  int ksplit;                          // K slices per output tile (1, 2 or 4)
   float* partial;                      // [tiles][ksplit][SK_PSZ] slice partials (ksplit > 1)
   unsigned* arrive;                    // [tiles] slice arrival counts, zero between launches
-  // BF16 form only:
+  // BF16 products only:
   const uint16_t* xs;                  // x in split form (xsplit_index), gain applied; null: FP32 x
   const float* ss_in; int n_ss;        // NORM with xs: [32][n_ss] partial sums of x^2 per row
   uint16_t* xs_out;                    // out again in split form for the next GEMM; null: none
@@ -58,138 +59,29 @@ constexpr int SK_ROWS = 32;             // rows covered (two 16-row MFMA tiles)
 typedef float sv4f __attribute__((ext_vector_type(4)));
 
 // out[r][o] for 16 outputs o of this workgroup and all rows r < R.  Lane l of
-// a wave holds weights of output o0 + l % 16 and rows (l % 16) (+16) of x for
-// VEC consecutive k at kb + VEC (l / 16); MFMA j pairs weight and x at the
-// same k, so every k of the block enters the sum exactly once.  Wave w takes
-// blocks w, w + W, ...; the next block's loads are in flight while one is
-// multiplied.  NORM: x is taken through RMSNorm -- the gain is applied per k,
-// the row's sum of squares is gathered on the way and 1 / rms scales the sum
-// at the end (out = inv_rms * sum_k w_k g_k x_k).  EPI is one of the GEMV
-// epilogues (store, bias, residual, SwiGLU).
-template <int EPI, typename WL, int W, bool NORM>
-__global__ __launch_bounds__(W * 64) void skinny_gemm_kernel(SkinnyArgs a) {
-  constexpr int NA = (EPI == EPI_SWIGLU) ? 2 : 1;
-  constexpr int VEC = WL::VEC;          // 4 (FP32) or 8 (BF16) k per lane per block
-  constexpr int BK = 4 * VEC;           // k per block
-  __shared__ float red[W][NA * 2 * 4][64];
-  __shared__ float ssq[NORM ? W : 1][2][64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int i16 = lane & 15, kq = lane >> 4;
-  const int o0 = blockIdx.x * 16;
-  const int o = min(o0 + i16, a.N - 1);
-  const void* wb;
-  int wr;
-  if (o < a.seg_rows[0]) { wb = a.w[0]; wr = o; }
-  else if (o < a.seg_rows[0] + a.seg_rows[1]) { wb = a.w[1]; wr = o - a.seg_rows[0]; }
-  else { wb = a.w[2]; wr = o - a.seg_rows[0] - a.seg_rows[1]; }
-  const size_t woff = (size_t)wr * a.K + VEC * kq;
-  const size_t w2off = (size_t)o * a.K + VEC * kq;
-  const float* xr0 = a.x + (size_t)min(i16, a.R - 1) * a.ldx + VEC * kq;
-  const float* xr1 = a.x + (size_t)min(16 + i16, a.R - 1) * a.ldx + VEC * kq;
-  const float* gp = NORM ? a.norm_w + VEC * kq : nullptr;
-  struct Stage { float w[NA][VEC], x0[VEC], x1[VEC], g[NORM ? VEC : 1]; };
-  auto load = [&](int kb, Stage& st) {
-    WL::load(wb, woff + kb, st.w[0]);
-    if constexpr (NA == 2) WL::load(a.w2, w2off + kb, st.w[NA - 1]);
-#pragma unroll
-    for (int j = 0; j < VEC; j += 4) {
-      const float4 p = *reinterpret_cast<const float4*>(xr0 + kb + j);
-      const float4 q = *reinterpret_cast<const float4*>(xr1 + kb + j);
-      st.x0[j] = p.x; st.x0[j + 1] = p.y; st.x0[j + 2] = p.z; st.x0[j + 3] = p.w;
-      st.x1[j] = q.x; st.x1[j + 1] = q.y; st.x1[j + 2] = q.z; st.x1[j + 3] = q.w;
-      if constexpr (NORM) {
-        const float4 g = *reinterpret_cast<const float4*>(gp + kb + j);
-        st.g[j] = g.x; st.g[j + 1] = g.y; st.g[j + 2] = g.z; st.g[j + 3] = g.w;
-      }
-    }
-  };
-  sv4f acc[NA][2];
-#pragma unroll
-  for (int n = 0; n < NA; ++n) acc[n][0] = acc[n][1] = sv4f{0.f, 0.f, 0.f, 0.f};
-  float ss0 = 0.f, ss1 = 0.f;
-  auto comp = [&](const Stage& st) {
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-      float x0 = st.x0[j], x1 = st.x1[j];
-      if constexpr (NORM) {
-        ss0 = fmaf(x0, x0, ss0);
-        ss1 = fmaf(x1, x1, ss1);
-        x0 *= st.g[j];
-        x1 *= st.g[j];
-      }
-#pragma unroll
-      for (int n = 0; n < NA; ++n) {
-        acc[n][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.w[n][j], x0, acc[n][0], 0, 0, 0);
-        acc[n][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(st.w[n][j], x1, acc[n][1], 0, 0, 0);
-      }
-    }
-  };
-  Stage sa, sb;
-  constexpr int STEP = W * BK;
-  int kb = wave * BK;
-  if (kb < a.K) load(kb, sa);
-  for (; kb < a.K; kb += 2 * STEP) {
-    const int k1 = kb + STEP, k2 = k1 + STEP;
-    if (k1 < a.K) load(k1, sb);
-    comp(sa);
-    if (k1 < a.K) {
-      if (k2 < a.K) load(k2, sa);
-      comp(sb);
-    }
-  }
-#pragma unroll
-  for (int n = 0; n < NA; ++n)
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) red[wave][(n * 2 + t) * 4 + v][lane] = acc[n][t][v];
-  if constexpr (NORM) { ssq[wave][0][lane] = ss0; ssq[wave][1][lane] = ss1; }
-  __syncthreads();
-  if (tid >= 512) return;
-  // thread -> (row tile t, v, lane): output o0 + 4 (lane / 16) + v, row 16 t + lane % 16
-  const int t = tid >> 8, v = (tid >> 6) & 3, l = tid & 63;
-  const int oo = o0 + 4 * (l >> 4) + v, r = 16 * t + (l & 15);
-  float c[NA];
-#pragma unroll
-  for (int n = 0; n < NA; ++n) {
-    float s = 0.f;
-#pragma unroll
-    for (int w = 0; w < W; ++w) s += red[w][(n * 2 + t) * 4 + v][l];
-    c[n] = s;
-  }
-  if constexpr (NORM) {
-    float ss = 0.f;
-#pragma unroll
-    for (int w = 0; w < W; ++w)
-#pragma unroll
-      for (int k4 = 0; k4 < 4; ++k4) ss += ssq[w][t][k4 * 16 + (l & 15)];
-    const float inv = 1.0f / sqrtf(ss / (float)a.K + a.eps);
-#pragma unroll
-    for (int n = 0; n < NA; ++n) c[n] *= inv;
-  }
-  if (oo < a.N && r < a.R) {
-    float y = c[0];
-    if constexpr (EPI == EPI_BIAS) y = y + a.bias[oo];
-    if constexpr (EPI == EPI_RESID) y = a.res[(size_t)r * a.ldr + oo] + y;
-    if constexpr (EPI == EPI_SWIGLU) {
-      if (a.pre_out) {
-        a.pre_out[(size_t)r * a.ld_pre + oo] = y;
-        a.pre_out[(size_t)r * a.ld_pre + a.N + oo] = c[NA - 1];
-      }
-      y = y / (1.0f + expf(-y)) * c[NA - 1];
-    }
-    a.out[(size_t)r * a.ldo + oo] = y;
-  }
-}
-
-// BF16 weights: the same GEMM on the BF16 matrix cores
-// (v_mfma_f32_16x16x32_bf16).  A lane's 8 consecutive BF16 weights are the A
-// fragment as loaded; each x value (times the norm gain) is split into x_hi =
-// bf16(x) and x_lo = bf16(x - x_hi), and both halves go through the MFMA, so
-// the products are exact in FP32 and x keeps ~16 mantissa bits (relative
-// error <= 2^-16).  Sums in FP32 as in the FP32 form.
-typedef __bf16 sbf8 __attribute__((ext_vector_type(8)));
-
+// a wave holds VEC consecutive k at kb + VEC (l / 16) of output o0 + l % 16's
+// weights and of rows (l % 16) (+ 16) of x, so every k of a block enters the
+// sum exactly once.  Wave w takes blocks w, w + W, ... of the slice.  NORM: x
+// is taken through RMSNorm -- the gain is applied per k, the row's sum of
+// squares is gathered on the way and 1 / rms scales the sum at the end (out =
+// inv_rms * sum_k w_k g_k x_k).  EPI is one of the GEMV epilogues (store, bias,
+// residual, SwiGLU).  TR: 16-row tiles of x (1 for R <= 16, which halves the x
+// loads and the products).  How the products are formed (MM):
+//   MM_SPLIT  BF16 weights, v_mfma_f32_16x16x32_bf16: each x value (times the
+//             norm gain) is split into x_hi = bf16(x) and x_lo = bf16(x -
+//             x_hi) and both go through the MFMA, so the products are exact in
+//             FP32 and x keeps ~16 mantissa bits (relative error <= 2^-16);
+//   MM_XS     the same with x already in split form (below);
+//   MM_F32    FP32 weights, v_mfma_f32_16x16x4f32: exact FP32 products;
+//   MM_WIDE   BF16 weights widened to FP32, the FP32 MFMA (the operator API,
+//             whose results are FP32 sums of the exact products).
+// MM_F32 and MM_WIDE take K a multiple of 4 and 8 (TAIL: not of the block).
+// What bounds it: at 8 to 32 rows the weights (HBM) in principle; in fact the
+// latency of a launch's loads, so every load of a slice is issued up front
+// where registers allow.  FP32 weights, 8 rows, the O / down projections of
+// the 0.6B shape (1024 x 2048 to 3072), mean per launch in the frame: 11.4 us
+// with one workgroup per tile over all of K and 32 rows of x, 5.6-6.0 us with K
+// over 4 slices and 16 rows; 16 utterances, BF16: unchanged.
 //
 // Split K (ksplit S > 1, for outputs too few to fill the GPU): the S slices of
 // an output tile are workgroups tile % 8 + 8 (S (tile / 8) + s), so all run on
@@ -208,6 +100,10 @@ typedef __bf16 sbf8 __attribute__((ext_vector_type(8)));
 // squares is the sum of the producer's per-tile partials (ss_in).  Outputs
 // can be written in split form for the next GEMM (xs_out, with that GEMM's
 // gain) together with their per-tile sums of squares (ss_out).
+enum { MM_SPLIT = 0, MM_XS = 1, MM_F32 = 2, MM_WIDE = 3 };
+typedef __bf16 sbf8 __attribute__((ext_vector_type(8)));
+typedef uint32_t su4 __attribute__((ext_vector_type(4)));   // native vectors: copies of HIP's uint4 / float4 structs went through scratch
+
 // XCC_ID hardware register of each workgroup (one 64-thread wave each): the
 // XCD it runs on.  Split K needs workgroups whose ids agree modulo 8 to share
 // an XCD (and so an L2).
@@ -217,16 +113,20 @@ __global__ __launch_bounds__(64) void xcd_probe_kernel(unsigned* ids) {
 }
 constexpr int XCD_PROBE_WGS = 2048;
 
-template <int EPI, int W, bool NORM, bool XS>
-__global__ __launch_bounds__(W * 64) void skinny_bf16_kernel(SkinnyArgs a) {
+template <int EPI, int W, bool NORM, int MM, int TR, bool TAIL = false>
+__global__ __launch_bounds__(W * 64) void skinny_kernel(SkinnyArgs a) {
+  constexpr bool XS = MM == MM_XS, WF = MM == MM_F32, EXACT = MM >= MM_F32;
   static_assert(!XS || W == 8, "split input: one thread per (row, 16th of the partial sums)");
+  static_assert(!TAIL || EXACT, "the BF16 products take whole blocks");
+  static_assert(W * 64 >= 256 * TR, "one thread per output");
   constexpr int NA = (EPI == EPI_SWIGLU) ? 2 : 1;
-  constexpr int BK = 32;                // k per block: 8 per lane
+  constexpr int VEC = WF ? 4 : 8;       // k per lane and block
+  constexpr int BK = 4 * VEC;           // k per block
   constexpr bool XNORM = NORM && !XS;   // gain and sum of squares taken from FP32 x here
-  __shared__ float red[W][NA * 2 * 4][64];
-  __shared__ float ssq[XNORM ? W : 1][2][64];
+  __shared__ float red[W][NA * TR * 4][64];
+  __shared__ float ssq[XNORM ? W : 1][TR][64];
   __shared__ float ssr[XS_ROWS];
-  __shared__ float sso[2][4][64];
+  __shared__ float sso[TR][4][64];
   __shared__ int last_slice;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i16 = lane & 15, kq = lane >> 4;
@@ -247,68 +147,133 @@ __global__ __launch_bounds__(W * 64) void skinny_bf16_kernel(SkinnyArgs a) {
   if (o < a.seg_rows[0]) { wb = a.w[0]; wr = o; }
   else if (o < a.seg_rows[0] + a.seg_rows[1]) { wb = a.w[1]; wr = o - a.seg_rows[0]; }
   else { wb = a.w[2]; wr = o - a.seg_rows[0] - a.seg_rows[1]; }
-  const uint16_t* wp = static_cast<const uint16_t*>(wb) + (size_t)wr * a.K + 8 * kq;
-  const uint16_t* w2p = NA == 2 ? static_cast<const uint16_t*>(a.w2) + (size_t)o * a.K + 8 * kq : nullptr;
-  const float* xr0 = a.x + (size_t)min(i16, a.R - 1) * a.ldx + 8 * kq;
-  const float* xr1 = a.x + (size_t)min(16 + i16, a.R - 1) * a.ldx + 8 * kq;
-  const float* gp = XNORM ? a.norm_w + 8 * kq : nullptr;
-  const uint4* xsp = XS ? reinterpret_cast<const uint4*>(a.xs) + lane : nullptr;
-  struct StageF { uint4 w[NA]; float4 x0[2], x1[2], g[XNORM ? 2 : 1]; };
-  struct StageS { uint4 w[NA]; uint4 xs[4]; };   // hi/lo of row tiles 0 and 1
+  constexpr int WES = WF ? 4 : 2;       // bytes of a weight
+  const char* wp = static_cast<const char*>(wb) + ((size_t)wr * a.K + VEC * kq) * WES;
+  const char* w2p = NA == 2 ? static_cast<const char*>(a.w2) + ((size_t)o * a.K + VEC * kq) * WES : nullptr;
+  const float* xr[TR];
+#pragma unroll
+  for (int t = 0; t < TR; ++t) xr[t] = a.x + (size_t)min(16 * t + i16, a.R - 1) * a.ldx + VEC * kq;
+  const float* gp = XNORM ? a.norm_w + VEC * kq : nullptr;
+  const su4* xsp = XS ? reinterpret_cast<const su4*>(a.xs) + lane : nullptr;
+  constexpr int NX = VEC / 4;           // float4 of x per lane, block and row tile
+  struct StageF { su4 w[NA]; sv4f x[TR][NX], g[XNORM ? NX : 1]; };
+  struct StageS { su4 w[NA]; su4 xs[2 * TR]; };   // hi/lo of each row tile
   using Stage = typename std::conditional<XS, StageS, StageF>::type;
-  auto load = [&](int kb, Stage& st) {
-    st.w[0] = *reinterpret_cast<const uint4*>(wp + kb);
-    if constexpr (NA == 2) st.w[NA - 1] = *reinterpret_cast<const uint4*>(w2p + kb);
+  auto load = [&](int kb, Stage& st) __attribute__((always_inline)) {
+    int off = kb;                       // TAIL: lanes past K re-read K's last elements, zeroed below
+    bool in = true;
+    if constexpr (TAIL) {
+      in = kb + VEC * kq < a.K;
+      off = min(kb, a.K - VEC - VEC * kq);
+    }
+    st.w[0] = *reinterpret_cast<const su4*>(wp + (ptrdiff_t)off * WES);
+    if constexpr (NA == 2) st.w[NA - 1] = *reinterpret_cast<const su4*>(w2p + (ptrdiff_t)off * WES);
     if constexpr (XS) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) st.xs[j] = xsp[((size_t)(kb >> 5) * 4 + j) * 64];
+      for (int j = 0; j < 2 * TR; ++j) st.xs[j] = xsp[((size_t)(kb >> 5) * 4 + j) * 64];
     } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        st.x0[h] = *reinterpret_cast<const float4*>(xr0 + kb + 4 * h);
-        st.x1[h] = *reinterpret_cast<const float4*>(xr1 + kb + 4 * h);
-        if constexpr (XNORM) st.g[h] = *reinterpret_cast<const float4*>(gp + kb + 4 * h);
+      for (int h = 0; h < NX; ++h) {
+#pragma unroll
+        for (int t = 0; t < TR; ++t) {
+          st.x[t][h] = *reinterpret_cast<const sv4f*>(xr[t] + off + 4 * h);
+          if constexpr (TAIL) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st.x[t][h][i] = in ? st.x[t][h][i] : 0.f;
+          }
+        }
+        if constexpr (XNORM) st.g[h] = *reinterpret_cast<const sv4f*>(gp + off + 4 * h);
+      }
+    }
+    if constexpr (TAIL) {
+#pragma unroll
+      for (int n = 0; n < NA; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) st.w[n][i] = in ? st.w[n][i] : 0u;
+    }
+  };
+  // Exact products: four sums, of k = 0, 1, 2, 3 mod 4, flushed into a total
+  // every 4 stages: chains of at most 32 (FP32: 16) products keep the sums'
+  // rounding below the GEMV kernels' (one chain over a wave's K: twice theirs).
+  constexpr int NACC = EXACT ? 4 : 1;
+  sv4f accs[NACC][NA][TR], tot[EXACT ? NA : 1][EXACT ? TR : 1];
+#pragma unroll
+  for (int n = 0; n < NA; ++n)
+#pragma unroll
+    for (int t = 0; t < TR; ++t) {
+#pragma unroll
+      for (int c = 0; c < NACC; ++c) accs[c][n][t] = sv4f{0.f, 0.f, 0.f, 0.f};
+      if constexpr (EXACT) tot[n][t] = sv4f{0.f, 0.f, 0.f, 0.f};
+    }
+  auto flush = [&]() __attribute__((always_inline)) {
+    if constexpr (EXACT) {
+#pragma unroll
+      for (int n = 0; n < NA; ++n)
+#pragma unroll
+        for (int t = 0; t < TR; ++t) {
+          tot[n][t] += (accs[0][n][t] + accs[1 % NACC][n][t]) + (accs[2 % NACC][n][t] + accs[3 % NACC][n][t]);
+#pragma unroll
+          for (int c = 0; c < NACC; ++c) accs[c][n][t] = sv4f{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
+  float ssx[TR] = {};
+  // this lane's x of row tile t, gain applied (XNORM: its squares gathered first)
+  auto xval = [&](const auto& st, int t, float (&v)[VEC]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < NX; ++h) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[4 * h + i] = st.x[t][h][i];
+        if constexpr (XNORM) {
+          ssx[t] = fmaf(v[4 * h + i], v[4 * h + i], ssx[t]);
+          v[4 * h + i] *= st.g[h][i];
+        }
       }
     }
   };
-  sv4f acc[NA][2];
+  auto comp = [&](const Stage& st) __attribute__((always_inline)) {
+    if constexpr (EXACT) {
+      float v[TR][VEC];
 #pragma unroll
-  for (int n = 0; n < NA; ++n) acc[n][0] = acc[n][1] = sv4f{0.f, 0.f, 0.f, 0.f};
-  float ss0 = 0.f, ss1 = 0.f;
-  auto split = [&](const float4 (&xv)[2], const float4 (&gv)[XNORM ? 2 : 1], float& ss, sbf8& hi, sbf8& lo) {
-    const float v[8] = {xv[0].x, xv[0].y, xv[0].z, xv[0].w, xv[1].x, xv[1].y, xv[1].z, xv[1].w};
+      for (int t = 0; t < TR; ++t) xval(st, t, v[t]);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float x = v[j];
-      if constexpr (XNORM) {
-        const float g[8] = {gv[0].x, gv[0].y, gv[0].z, gv[0].w, gv[XNORM ? 1 : 0].x, gv[XNORM ? 1 : 0].y,
-                            gv[XNORM ? 1 : 0].z, gv[XNORM ? 1 : 0].w};
-        ss = fmaf(x, x, ss);
-        x *= g[j];
-      }
-      const __bf16 h = (__bf16)x;
-      hi[j] = h;
-      lo[j] = (__bf16)(x - (float)h);
-    }
-  };
-  auto comp = [&](const Stage& st) {
-    sbf8 h0, l0, h1, l1;
-    if constexpr (XS) {
-      h0 = __builtin_bit_cast(sbf8, st.xs[0]);
-      l0 = __builtin_bit_cast(sbf8, st.xs[1]);
-      h1 = __builtin_bit_cast(sbf8, st.xs[2]);
-      l1 = __builtin_bit_cast(sbf8, st.xs[3]);
+      for (int j = 0; j < VEC; ++j)
+#pragma unroll
+        for (int n = 0; n < NA; ++n) {
+          const uint32_t ww = st.w[n][WF ? j % 4 : j / 2];
+          const float wv = __uint_as_float(WF ? ww : j & 1 ? ww & 0xffff0000u : ww << 16);
+#pragma unroll
+          for (int t = 0; t < TR; ++t)
+            accs[j % NACC][n][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, v[t][j], accs[j % NACC][n][t], 0, 0, 0);
+        }
     } else {
-      split(st.x0, st.g, ss0, h0, l0);
-      split(st.x1, st.g, ss1, h1, l1);
-    }
+      sbf8 hi[TR], lo[TR];
 #pragma unroll
-    for (int n = 0; n < NA; ++n) {
-      const sbf8 wa = __builtin_bit_cast(sbf8, st.w[n]);
-      acc[n][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, h0, acc[n][0], 0, 0, 0);
-      acc[n][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, l0, acc[n][0], 0, 0, 0);
-      acc[n][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, h1, acc[n][1], 0, 0, 0);
-      acc[n][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, l1, acc[n][1], 0, 0, 0);
+      for (int t = 0; t < TR; ++t) {
+        if constexpr (XS) {
+          hi[t] = __builtin_bit_cast(sbf8, st.xs[2 * t]);
+          lo[t] = __builtin_bit_cast(sbf8, st.xs[2 * t + 1]);
+        } else {
+          float v[VEC];
+          xval(st, t, v);
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) {
+            const __bf16 h = (__bf16)v[j];
+            hi[t][j] = h;
+            lo[t][j] = (__bf16)(v[j] - (float)h);
+          }
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < NA; ++n) {
+        const sbf8 wa = __builtin_bit_cast(sbf8, st.w[n]);
+#pragma unroll
+        for (int t = 0; t < TR; ++t) {
+          accs[0][n][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, hi[t], accs[0][n][t], 0, 0, 0);
+          accs[0][n][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, lo[t], accs[0][n][t], 0, 0, 0);
+        }
+      }
     }
   };
   // Split input with NORM: the producer's partial sums of squares of row
@@ -327,8 +292,8 @@ __global__ __launch_bounds__(W * 64) void skinny_bf16_kernel(SkinnyArgs a) {
   }
   // Epilogue operands of this thread's output (row r, column oo), loaded at
   // entry: they do not depend on the sums.
-  const bool et = tid < 512;            // threads 0..511 own one (row tile, v, lane) each
-  const int t = (tid >> 8) & 1, v = (tid >> 6) & 3, l = tid & 63;
+  const bool et = tid < 256 * TR;       // these threads own one (row tile, v, lane) each
+  const int t = TR == 2 ? (tid >> 8) & 1 : 0, v = (tid >> 6) & 3, l = tid & 63;
   const int oo = o0 + 4 * (l >> 4) + v, r = 16 * t + (l & 15);
   const bool ok = et && oo < a.N && r < a.R;
   float epi_in = 0.f;
@@ -337,45 +302,68 @@ __global__ __launch_bounds__(W * 64) void skinny_bf16_kernel(SkinnyArgs a) {
   // the split-form output's gain too (index clamped: no branch around the load)
   const float gain_in = a.xs_gain ? a.xs_gain[min(oo, a.N - 1)] : 1.f;
   constexpr int STEP = W * BK;
-  // This wave's stages: k = kw0 + i * STEP for i < nst.  Up to 4 stages
-  // (every K / split of the 0.6B shapes) the wave issues all of its loads up
-  // front, in straight-line code for its exact stage count, then multiplies
-  // the stages in order: each multiply waits for its own stage only.  (In a
-  // loop with conditional loads the compiler cannot count the loads in flight
-  // and waited for all of them.)  Longer slices use the two-stage ring.
+  // This wave's stages: k = kw0 + i * STEP for i < nst.  Up to UP stages (8, or 4
+  // where a stage is wide; nearly every slice of the 0.6B shapes) the wave
+  // issues all of its loads up front, in straight-line code for its exact
+  // stage count, then multiplies the stages in order: each multiply waits for
+  // its own stage only.  (In a loop with conditional loads the compiler cannot
+  // count the loads in flight and waited for all of them.)  Longer slices go
+  // in chunks of UP / 2 stages, the next chunk's loads in flight under this one's
+  // products, then the remainder up front.
   const int kw0 = kbeg + wave * BK;
   const int nst = kw0 < kend ? (kend - kw0 + STEP - 1) / STEP : 0;
-  auto upfront = [&](auto nc) {
+  constexpr int SREG = XS ? 4 * NA + 8 * TR : (NA + (TR + (XNORM ? 1 : 0)) * NX) * 4;   // registers of a stage
+  constexpr int UP = SREG > 20 || (MM <= MM_XS && TR == 2) ? 4 : 8, CH = UP / 2;
+  auto upfront = [&](int k0, auto nc) __attribute__((always_inline)) {
     constexpr int NC = decltype(nc)::value;
     Stage st[NC];
 #pragma unroll
-    for (int i = 0; i < NC; ++i) load(kw0 + i * STEP, st[i]);
+    for (int i = 0; i < NC; ++i) load(k0 + i * STEP, st[i]);
     asm volatile("" ::: "memory");   // not sunk towards the multiplies
 #pragma unroll
-    for (int i = 0; i < NC; ++i) comp(st[i]);
-  };
-  if (nst == 1) {
-    upfront(std::integral_constant<int, 1>{});
-  } else if (nst == 2) {
-    upfront(std::integral_constant<int, 2>{});
-  } else if (nst == 3) {
-    upfront(std::integral_constant<int, 3>{});
-  } else if (nst == 4) {
-    upfront(std::integral_constant<int, 4>{});
-  } else if (nst > 4) {
-    Stage sa, sb;
-    int kb = kw0;
-    load(kb, sa);
-    for (; kb < kend; kb += 2 * STEP) {
-      const int k1 = kb + STEP, k2 = k1 + STEP;
-      if (k1 < kend) load(k1, sb);
-      comp(sa);
-      if (k1 < kend) {
-        if (k2 < kend) load(k2, sa);
-        comp(sb);
-      }
+    for (int i = 0; i < NC; ++i) {
+      comp(st[i]);
+      if (i % 4 == 3 || i == NC - 1) flush();
     }
+  };
+  auto rest = [&](int k0, int n) __attribute__((always_inline)) {
+    if (n == 1) upfront(k0, std::integral_constant<int, 1>{});
+    else if (n == 2) upfront(k0, std::integral_constant<int, 2>{});
+    else if (n == 3) upfront(k0, std::integral_constant<int, 3>{});
+    else if (n == 4) upfront(k0, std::integral_constant<int, 4>{});
+    if constexpr (UP == 8) {
+      if (n == 5) upfront(k0, std::integral_constant<int, 5>{});
+      else if (n == 6) upfront(k0, std::integral_constant<int, 6>{});
+      else if (n == 7) upfront(k0, std::integral_constant<int, 7>{});
+      else if (n == 8) upfront(k0, std::integral_constant<int, 8>{});
+    }
+  };
+  int done = 0;                         // stages already multiplied
+  if (nst > UP) {
+    Stage sa[CH], sb[CH];
+    auto load4 = [&](int c, Stage (&st)[CH]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) load(kw0 + (c * CH + i) * STEP, st[i]);
+      asm volatile("" ::: "memory");
+    };
+    auto comp4 = [&](const Stage (&st)[CH]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) comp(st[i]);
+      flush();
+    };
+    const int nch = nst / CH;
+    load4(0, sa);
+    for (int c = 0;; c += 2) {
+      if (c + 1 >= nch) { comp4(sa); break; }
+      load4(c + 1, sb);
+      comp4(sa);
+      if (c + 2 >= nch) { comp4(sb); break; }
+      load4(c + 2, sa);
+      comp4(sb);
+    }
+    done = nch * CH;
   }
+  rest(kw0 + done * STEP, nst - done);
   // The row's sum of squares is needed only by the epilogue: summed after the
   // stream, so waiting for the partials never holds back a stage's loads.
   if constexpr (XS && NORM) {
@@ -391,18 +379,30 @@ __global__ __launch_bounds__(W * 64) void skinny_bf16_kernel(SkinnyArgs a) {
 #pragma unroll
   for (int n = 0; n < NA; ++n)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < TR; ++t)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) red[wave][(n * 2 + t) * 4 + v][lane] = acc[n][t][v];
-  if constexpr (XNORM) { ssq[wave][0][lane] = ss0; ssq[wave][1][lane] = ss1; }
+      for (int v = 0; v < 4; ++v)
+        red[wave][(n * TR + t) * 4 + v][lane] = EXACT ? tot[EXACT ? n : 0][EXACT ? t : 0][v] : accs[0][n][t][v];
+  if constexpr (XNORM) {
+#pragma unroll
+    for (int t = 0; t < TR; ++t) ssq[wave][t][lane] = ssx[t];
+  }
   __syncthreads();
-  // With 16 waves the upper half only takes part in the barriers.
+  // Waves past the output threads only take part in the barriers.
   float c[NA];
 #pragma unroll
   for (int n = 0; n < NA; ++n) {
     float sacc = 0.f;
+    if constexpr (EXACT && W % 4 == 0) {   // in groups of 4 waves, for the sums' rounding
 #pragma unroll
-    for (int w = 0; w < W; ++w) sacc += red[w][(n * 2 + t) * 4 + v][l];
+      for (int w = 0; w < W; w += 4) {
+        const int i = (n * TR + t) * 4 + v;
+        sacc += (red[w][i][l] + red[w + 1][i][l]) + (red[w + 2][i][l] + red[w + 3][i][l]);
+      }
+    } else {
+#pragma unroll
+      for (int w = 0; w < W; ++w) sacc += red[w][(n * TR + t) * 4 + v][l];
+    }
     c[n] = sacc;
   }
   float ss = 0.f;
@@ -544,4 +544,65 @@ __global__ __launch_bounds__(W * 64) void skinny_bf16_kernel(SkinnyArgs a) {
   }
 }
 
+
+// K over 4 or 2 workgroups per output tile when the tiles alone would fill
+// fewer than 256 CUs (tiles a multiple of 8, slices whole blocks).
+template <int EPI, bool NORM, int MM, int TR>
+inline hipError_t launch_skinny_t(SkinnyArgs a, bool allow_split, hipStream_t st) {
+  const int tiles = (a.N + 15) / 16;
+  constexpr int BK = MM == MM_F32 ? 16 : 32;
+  a.ksplit = 1;
+  if (allow_split && tiles % 8 == 0) {
+    if (tiles <= 64 && a.K % (4 * BK) == 0) a.ksplit = 4;
+    else if (tiles <= 128 && a.K % (2 * BK) == 0) a.ksplit = 2;
+  }
+  static_assert(SK_MAX_SPLIT >= 4, "the kernel's split-K merge covers the splits chosen here");
+  hipLaunchKernelGGL((skinny_kernel<EPI, 8, NORM, MM, TR>), dim3(tiles * a.ksplit), dim3(8 * 64), 0, st, a);
+  return hipGetLastError();
+}
+// A GEMM of at most 32 rows in the engine's forms: split products with BF16
+// weights (x in split form when a.xs is given), exact FP32 ones otherwise.
+template <int EPI, bool NORM>
+inline hipError_t launch_skinny_w(bool bf16, const SkinnyArgs& a, bool allow_split, hipStream_t st) {
+  const bool one = a.R <= 16;
+  if (!bf16) return one ? launch_skinny_t<EPI, NORM, MM_F32, 1>(a, allow_split, st)
+                        : launch_skinny_t<EPI, NORM, MM_F32, 2>(a, allow_split, st);
+  if (a.xs) return one ? launch_skinny_t<EPI, NORM, MM_XS, 1>(a, allow_split, st)
+                       : launch_skinny_t<EPI, NORM, MM_XS, 2>(a, allow_split, st);
+  return one ? launch_skinny_t<EPI, NORM, MM_SPLIT, 1>(a, allow_split, st)
+             : launch_skinny_t<EPI, NORM, MM_SPLIT, 2>(a, allow_split, st);
+}
+
+// The operator API's projections of at most 32 rows: exact products, any N, K
+// a multiple of 8.  SwiGLU of up to 16 rows in workgroups of 4 waves (three per
+// CU, so one loads while another multiplies: 7 rows, BF16 2 x 6144 x 2048, 18.3 us
+// against 30.4 us with 8 waves), the rest, with half the tiles, of 8 (2048 x
+// 6144: 15.2 us against 19.6 with 4 and 22.5 with 16).
+template <int EPI, int MM, int TR, bool TAIL>
+inline hipError_t launch_rows_t(const SkinnyArgs& a, hipStream_t st) {
+  constexpr int W = EPI == EPI_SWIGLU && TR == 1 ? 4 : 8;
+  hipLaunchKernelGGL((skinny_kernel<EPI, W, false, MM, TR, TAIL>), dim3((a.N + 15) / 16), dim3(W * 64), 0, st, a);
+  return hipGetLastError();
+}
+template <int EPI, int MM>
+inline hipError_t launch_rows_m(const SkinnyArgs& a, hipStream_t st) {
+  const bool tail = a.K % (MM == MM_F32 ? 16 : 32) != 0;
+  if (a.R <= 16) return tail ? launch_rows_t<EPI, MM, 1, true>(a, st) : launch_rows_t<EPI, MM, 1, false>(a, st);
+  return tail ? launch_rows_t<EPI, MM, 2, true>(a, st) : launch_rows_t<EPI, MM, 2, false>(a, st);
+}
+template <int EPI>
+inline hipError_t launch_rows(bool bf16, SkinnyArgs a, hipStream_t st) {
+  a.ksplit = 1;
+  return bf16 ? launch_rows_m<EPI, MM_WIDE>(a, st) : launch_rows_m<EPI, MM_F32>(a, st);
+}
+inline SkinnyArgs skinny_args(const void* w, int N, int K, const float* x, int ldx, float* out, int ldo, int R) {
+  SkinnyArgs a{};
+  a.w[0] = w;
+  a.seg_rows[0] = N;
+  a.x = x; a.ldx = ldx; a.out = out; a.ldo = ldo;
+  a.R = R; a.N = N; a.K = K;
+  return a;
+}
+
+}  // namespace
 }  // namespace sk

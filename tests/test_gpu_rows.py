@@ -1,0 +1,107 @@
+"""Projections of many rows: the operator API's SwiGLU, down + residual and
+classifier for 1 to 70 rows (one and two 16-row tiles, several launches), with
+output counts that leave a partial tile of 16 and K that ends inside a block
+(32 of K per block with BF16 weights, 16 with FP32), and the engine's FP32
+many-row path with its K slices.
+
+Operator tolerance: relative to the output's largest value; exact products
+summed in FP32 over up to 3,080 terms in another order: ~sqrt(K) 2^-24 = 3e-6,
+2e-5 with the largest value only a few times a typical one."""
+
+import numpy as np
+import pytest
+
+import oracle.model as om
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(got, ref):
+    return float(np.abs(np.asarray(got, np.float64) - ref).max() / np.abs(ref).max())
+
+
+@pytest.mark.parametrize("B", [3, 4, 5, 16, 17, 32, 33, 70])
+@pytest.mark.parametrize("K,N", [(1024, 2051), (3072, 1024), (8, 17), (72, 40), (1000, 96), (3080, 48), (2048, 3000)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_rows_ops_match_float64(hip_device, B, K, N, bf16):
+    import torch
+
+    from soraku_amd import ops
+
+    rng = np.random.default_rng(B * 7919 + K)
+    dt = torch.bfloat16 if bf16 else torch.float32
+
+    def mat(*s):
+        w = rng.standard_normal(s, dtype=np.float32) * np.float32(0.05)
+        return om.round_bf16(w) if bf16 else w
+
+    def dev(x, d=None):
+        t = torch.from_numpy(x).to(hip_device)
+        return t if d is None else t.to(d)
+
+    print(f"rows B={B} K={K} N={N} bf16={bf16}", flush=True)
+    x, res, bias = (rng.standard_normal(s, dtype=np.float32) for s in ((B, K), (B, N), (N,)))
+    wg, wu = mat(N, K), mat(N, K)
+    x64, g64 = x.astype(np.float64), wg.T.astype(np.float64)
+    got = ops.classifier_gemv(B, N, K)(dev(x), dev(wg, dt), dev(bias)).cpu().numpy()
+    assert _rel(got, x64 @ g64 + bias) < 2e-5
+    got = ops.down_residual_gemv(B, N, K)(dev(x), dev(wg, dt), dev(res)).cpu().numpy()
+    assert _rel(got, x64 @ g64 + res) < 2e-5
+    got = ops.swiglu_gemv(B, N, K)(dev(x), dev(wg, dt), dev(wu, dt)).cpu().numpy()
+    assert _rel(got, om.silu(x64 @ g64) * (x64 @ wu.T.astype(np.float64))) < 2e-5
+
+
+def test_rows_op_keeps_bad_rows_apart(hip_device):
+    """NaN and infinity in one activation row stay in that row."""
+    import torch
+
+    from soraku_amd import ops
+
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((7, 104), dtype=np.float32)
+    x[2, 5], x[6, 100] = np.nan, np.inf
+    w = torch.from_numpy(rng.standard_normal((33, 104), dtype=np.float32)).to(hip_device)
+    b = torch.zeros(33, device=hip_device)
+    got = ops.classifier_gemv(7, 33, 104)(torch.from_numpy(x).to(hip_device), w, b).cpu().numpy()
+    ok = [0, 1, 3, 4, 5]
+    ref = x[ok].astype(np.float64) @ w.cpu().numpy().T.astype(np.float64)
+    assert np.isfinite(got[ok]).all() and _rel(got[ok], ref) < 2e-5
+    assert np.isnan(got[2]).all() and not np.isfinite(got[6]).any()
+
+
+@pytest.mark.parametrize("utts", [3, 8, 16])
+def test_fp32_many_rows_match_oracle(hip_device, utts):
+    """FP32 weights, 6 to 32 decode rows at a width whose O, down and depth
+    down projections take 4 K slices: two teacher-forced frames' logits."""
+    from oracle.generate import Record, generate
+    from oracle.sampler import apply_masks
+    from soraku_amd import GraphFrameEngine
+    from soraku_amd.config import DecodeShape
+
+    s = om.Shape(d_model=1024, n_layers=2, trunk_inter=3072, n_codebooks=4, codebook_size=61, text_vocab=512)
+    w = om.synthetic_weights(s, 9, norm_gain_std=0.1, bias_std=0.02)
+    rng = np.random.default_rng(utts)
+    items = [(rng.integers(0, 512, 5 + i), np.array([1], np.int64), rng.integers(0, 61, (3 + i, 4))) for i in range(utts)]
+    forced = rng.integers(0, 61, (2, utts, 4))
+    e = GraphFrameEngine(device=hip_device, max_cache_len=64, cfg_scale=1.5, batch=2, state_dict=w,
+                         shape=DecodeShape(**{k: getattr(s, k) for k in DecodeShape.__dataclass_fields__}), n_utts=utts)
+    e.set_debug(True)
+    e.prefill_utterances(items)
+    e.capture()
+    got = []
+    for f in range(2):
+        print(f"fp32 frame {f} of {utts} utterances", flush=True)
+        got.append(e.step_frame(mask_eos_q0=True, forced_codes=forced[f], return_logits=True)[1])
+    e.close()
+    m = om.OracleModel(s, w, np.float64)
+    for u in (0, utts // 2, utts - 1):
+        text, uncond, prompt = items[u]
+        rec = Record()
+        generate(m, input_ids=text, prompt_codes=prompt, uncond_input_ids=uncond, max_new_frames=2, min_new_frames=2,
+                 temperature=0.0, cfg_scale=1.5, batched=True, record=rec, forced_codes=forced[:, u])
+        ref = [np.stack([apply_masks(x, q=q, frame_index=f, min_new_frames=2, bos_id=s.bos_id, eos_id=s.eos_id,
+                                     pad_id=s.pad_id) for q, x in enumerate(fr)]) for f, fr in enumerate(rec.merged)]
+        for f in range(2):
+            fin = np.isfinite(ref[f])
+            assert (np.isfinite(got[f][u]) == fin).all()
+            assert np.abs(got[f][u][fin] - ref[f][fin]).max() / np.abs(ref[f][fin]).max() < 5e-5
