@@ -153,10 +153,10 @@ int sk_set_sampling(sk_engine* e, float cfg_scale, float temperature, int32_t to
 int sk_set_debug(sk_engine* e, int32_t record_logits);
 
 /* Capture one whole frame (16 depth steps + sampling + frame embedding +
- * trunk step) as one hipGraph.  With one utterance with CFG at the
- * Qwen3-0.6B shape with FP32 weights or the Qwen3-1.7B shape with BF16
- * weights, capture also derives the depth steps' code tables from the bound
- * codebook table, depth norm_in gain and gate/up weights
+ * trunk step) as one hipGraph.  With one utterance (with or without CFG) at
+ * the depth widths of the Qwen3-0.6B or Qwen3-1.7B shape, and with more than 4
+ * decode rows, capture also derives the depth steps' code tables from the
+ * bound codebook table, depth norm_in gain and gate/up weights
  * ((Q-1) x V x 2 x depth_inner floats: 0.5 GB / 1.0 GB); those weights must
  * not change afterwards. */
 int sk_capture(sk_engine* e);
@@ -190,8 +190,8 @@ void* sk_stream(sk_engine* e);
 int32_t sk_frames_done(sk_engine* e);
 /* Diagnostic with no counterpart in the reference (which has one decode
  * path): 1 when the engine runs its trunk as XCD-resident layers (two
- * launches per layer; one utterance with CFG at the Qwen3-0.6B or, with BF16
- * weights, Qwen3-1.7B shape, on a device of 256 CUs, unless
+ * launches per layer; one or two decode rows at the Qwen3-0.6B or Qwen3-1.7B
+ * trunk shape, on a device of 256 CUs, unless
  * SORAKU_XCD_LAYERS=0 was set at sk_create), 0 when it runs the per-op layer
  * kernels, -1 for a NULL engine.  For tests and profiling. */
 int32_t sk_xcd_layers(sk_engine* e);

@@ -471,7 +471,7 @@ hipError_t launch_attn_stream(sk_engine* e, const AttnArgs& at) {
   return e->c.kv_dtype == SK_BF16 ? launch_attn_stream_kt<uint16_t>(e, at) : launch_attn_stream_kt<float>(e, at);
 }
 
-// XCD-resident layers (sk_layer.h): one utterance with CFG, 16 q / 8 KV heads
+// XCD-resident layers (sk_layer.h): one or two decode rows, 16 q / 8 KV heads
 // of 128, at the Qwen3-0.6B trunk shape (d 1024, SwiGLU 3072) or the
 // Qwen3-1.7B one (d 2048, SwiGLU 6144), FP32 or BF16 weights and cache.
 bool lx_fits(const sk_engine* e) {
@@ -481,7 +481,7 @@ bool lx_fits(const sk_engine* e) {
   // next frame's first-layer target, which the frame's last launch must zero
   // after every workgroup has read the whole output: one kernel cannot order
   // that, so such trunks keep the five-kernel layers.
-  return e->rows == LX_M && !e->wide && e->attn_splits == 0 && c.n_kv_heads == LX_HKV && c.n_q_heads == LX_HQ &&
+  return e->rows <= LX_M && !e->wide && e->attn_splits == 0 && c.n_kv_heads == LX_HKV && c.n_q_heads == LX_HQ &&
          c.head_dim == LX_HD && shape && e->max_chunks <= LX_MAXCH && c.n_layers % 3 != 2;
 }
 
@@ -501,7 +501,7 @@ hipError_t launch_lx(int d, bool first, const LxArgs& A, const LxArgs& C, hipStr
 
 // Fixed-point accumulator k % 3 of the XCD-resident layers (sk_layer.h).
 unsigned long long* lx_acc(const sk_engine* e, int k) {
-  return e->lx_acc + (size_t)(k % 3) * e->rows * e->c.d_model;
+  return e->lx_acc + (size_t)(k % 3) * LX_M * e->c.d_model;
 }
 
 // Each layer as two launches: attention half (x -> q/k/v -> attention -> O
@@ -527,7 +527,7 @@ hipError_t enqueue_trunk_lx(sk_engine* e) {
     A.vc = e->vc + (size_t)l * kv_layer_bytes(e);
     A.rope = e->rope; A.kv_len = e->kv_len; A.active = e->active;
     A.flags = e->lx_flags; A.err = e->lx_err;
-    A.max_ctx = c.max_ctx; A.max_chunks = e->max_chunks;
+    A.max_ctx = c.max_ctx; A.max_chunks = e->max_chunks; A.kv_rows = e->rows;
     A.eps = c.trunk_eps; A.scale = 1.0f / sqrtf((float)c.head_dim);
     A.spin_ticks = e->spin_ticks;
     LxArgs C = A;
@@ -674,7 +674,7 @@ hipError_t launch_g1(sk_engine* e) {
   DepthArgs g = depth_args(e);
   g.g_out = e->gbuf[0];
   SampleArgs s{};
-  return launch_depth_step<0>(e->c.weight_dtype, e->c.d_model, s, g, 0, e->stream);
+  return launch_depth_step<0>(e->c.weight_dtype, e->c.d_model, e->rows, s, g, 0, e->stream);
 }
 
 hipError_t enqueue_frame(sk_engine* e) {
@@ -711,7 +711,7 @@ hipError_t enqueue_frame(sk_engine* e) {
     for (int q = 0; q < c.n_codebooks; ++q) {
       if (q == 0) {   // G_1 is in gbuf[0]: from the previous frame's end, the prefill or the capture
         g.g_in = e->gbuf[0];
-        if ((err = launch_depth_step<1>(wt, d, s, g, 0, e->stream)) != hipSuccess) return err;
+        if ((err = launch_depth_step<1>(wt, d, M, s, g, 0, e->stream)) != hipSuccess) return err;
       } else {
         g.prefix_in = (q % 2 == 1) ? e->prefix : e->prefix2;
         g.prefix_out = (q % 2 == 1) ? e->prefix2 : e->prefix;
@@ -720,7 +720,7 @@ hipError_t enqueue_frame(sk_engine* e) {
         // the last codebook too: its G_{q+1} lands in gbuf[1], which codebook
         // 1 of the next frame rewrites before codebook 2 reads it (a variant
         // without that store ran ~1.3 us (0.6B) / ~2.5 us (1.7B) slower)
-        err = launch_depth_step<2>(wt, d, s, g, q, e->stream);
+        err = launch_depth_step<2>(wt, d, M, s, g, q, e->stream);
         if (err != hipSuccess) return err;
       }
       const void* tq = static_cast<const char*>(e->out_proj ? e->out_proj : e->table) + (size_t)q * V * d * tsz;
@@ -824,8 +824,8 @@ hipError_t enqueue_tail(sk_engine* e) {
     g.inv_freq = e->inv_freq; g.half = c.head_dim / 2; g.rope = e->rope;
     g.rope_tab = (const float2*)e->p_rope; g.tab_n = c.max_ctx + 1;
     SampleArgs s{};
-    return e->lx ? launch_depth_step<4>(c.weight_dtype, d, s, g, 0, e->stream)    // fixed-point trunk output
-                 : launch_depth_step<5>(c.weight_dtype, d, s, g, 0, e->stream);   // FP32 trunk output
+    return e->lx ? launch_depth_step<4>(c.weight_dtype, d, M, s, g, 0, e->stream)    // fixed-point trunk output
+                 : launch_depth_step<5>(c.weight_dtype, d, M, s, g, 0, e->stream);   // FP32 trunk output
   }
   hipLaunchKernelGGL(final_norm_kernel, dim3(M), dim3(NT), 0, e->stream, e->x,
                      e->lx ? reinterpret_cast<const long long*>(lx_acc(e, 2 * c.n_layers)) : nullptr,
@@ -1180,14 +1180,17 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
     return bail(SK_EHIP);
   }
   const size_t R = e->rows, d = c.d_model, Q = c.n_codebooks, V = c.audio_vocab;
-  ALLOC(e->x, R * d); ALLOC(e->hidden, R * d); ALLOC(e->prefix, R * d); ALLOC(e->prefix2, R * d);
+  // The XCD-resident layers always run two rows: with one, the second is an
+  // inactive row of zeros (RA rows of what they read per row; no cache).
+  const size_t RA = std::max<size_t>(R, LX_M);
+  ALLOC(e->x, RA * d); ALLOC(e->hidden, R * d); ALLOC(e->prefix, R * d); ALLOC(e->prefix2, R * d);
   ALLOC(e->abuf, R * d); ALLOC(e->ybuf, R * d);
   ALLOC(e->qkv, R * e->nqkv); ALLOC(e->attn, R * c.n_q_heads * c.head_dim);
   ALLOC(e->act, R * e->inner_max); ALLOC(e->logits, R * V);
   ALLOC(e->kc, (size_t)c.n_layers * kv_layer_bytes(e));
   ALLOC(e->vc, (size_t)c.n_layers * kv_layer_bytes(e));
   ALLOC(e->inv_freq, (size_t)c.head_dim / 2);
-  ALLOC(e->rope, R * (size_t)c.head_dim / 2);
+  ALLOC(e->rope, RA * (size_t)c.head_dim / 2);
   {
     const size_t nmax = std::max({(size_t)e->nqkv, (size_t)c.trunk_inter, (size_t)c.depth_inner,
                                   (size_t)c.audio_vocab, (size_t)c.d_model});
@@ -1197,14 +1200,14 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
     e->sk_tpart_bytes = (nmax / 16 + 1) * SK_MAX_SPLIT * SK_PSZ * sizeof(unsigned long long);
     ALLOC(e->sk_err, 1);
   }
-  ALLOC(e->part, R * c.n_q_heads * e->max_chunks * part_stride(c.head_dim));
+  ALLOC(e->part, RA * c.n_q_heads * e->max_chunks * part_stride(c.head_dim));
   const bool split_in = e->wide && c.weight_dtype == SK_BF16;
   if (split_in) {
     ALLOC(e->xs_x, xsplit_elems(d)); ALLOC(e->xs_attn, xsplit_elems(c.n_q_heads * c.head_dim));
     ALLOC(e->xs_act, xsplit_elems(e->inner_max)); ALLOC(e->xs_abuf, xsplit_elems(d)); ALLOC(e->xs_y, xsplit_elems(d));
     ALLOC(e->ss_x, (size_t)XS_ROWS * d / 16); ALLOC(e->ss_y, (size_t)XS_ROWS * d / 16);
   }
-  ALLOC(e->kv_len, R); ALLOC(e->pos, R); ALLOC(e->active, R); ALLOC(e->plen, R);
+  ALLOC(e->kv_len, RA); ALLOC(e->pos, RA); ALLOC(e->active, RA); ALLOC(e->plen, R);
   ALLOC(e->fc, 1);
   ALLOC(e->p_rope, (size_t)(c.max_ctx + 1) * (c.head_dim / 2));
   ALLOC(e->p_row_start, R);
@@ -1225,17 +1228,19 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
   hipError_t he = hipMemcpy(e->inv_freq, inv.data(), inv.size() * sizeof(float), hipMemcpyHostToDevice);
   if (he == hipSuccess) he = hipMemset(e->u_cur, 0, (size_t)c.n_utts * Q * sizeof(double));
   if (he == hipSuccess) he = hipMemset(e->flag_cur, 0, 2 * sizeof(int));
-  if (he == hipSuccess) he = hipMemset(e->x, 0, R * d * sizeof(float));
+  if (he == hipSuccess) he = hipMemset(e->x, 0, RA * d * sizeof(float));
+  if (he == hipSuccess) he = hipMemset(e->rope, 0, RA * (size_t)c.head_dim / 2 * sizeof(float2));
+  if (he == hipSuccess) he = hipMemset(e->active, 0, RA * sizeof(int));
   if (he == hipSuccess) he = hipMemset(e->prefix, 0, R * d * sizeof(float));
   if (he == hipSuccess) he = hipMemset(e->prefix2, 0, R * d * sizeof(float));
-  if (he == hipSuccess) he = hipMemset(e->kv_len, 0, R * sizeof(int));
+  if (he == hipSuccess) he = hipMemset(e->kv_len, 0, RA * sizeof(int));
   if (he == hipSuccess) he = hipMemset(e->sk_err, 0, sizeof(unsigned));
   if (he == hipSuccess) he = hipMemset(e->sk_tpart, 0, e->sk_tpart_bytes);   // tag 0 is never a launch's
   if (he == hipSuccess)
     he = hipMemset(e->sk_arrive, 0,
                    (std::max({(size_t)e->nqkv, (size_t)c.trunk_inter, (size_t)c.depth_inner, (size_t)c.audio_vocab,
                               (size_t)c.d_model}) / 16 + 1) * sizeof(unsigned));
-  if (he == hipSuccess) he = hipMemset(e->pos, 0, R * sizeof(int));
+  if (he == hipSuccess) he = hipMemset(e->pos, 0, RA * sizeof(int));
   if (split_in) {   // rows past R are never written; keep them finite
     uint16_t* xs[] = {e->xs_x, e->xs_attn, e->xs_act, e->xs_abuf, e->xs_y};
     const size_t xk[] = {d, (size_t)c.n_q_heads * c.head_dim, (size_t)e->inner_max, d, d};
@@ -1268,10 +1273,10 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
     e->lx = he == hipSuccess && mapped;
   }
   if (he == hipSuccess && e->lx) {
-    he = dalloc(&e->lx_acc, 3 * (size_t)R * d);
+    he = dalloc(&e->lx_acc, 3 * (size_t)LX_M * d);
     if (he == hipSuccess) he = dalloc(&e->lx_flags, (size_t)LX_XCDS * LX_FLAGS);
     if (he == hipSuccess) he = dalloc(&e->lx_err, 1);
-    const size_t nqkv = (size_t)R * (c.n_q_heads + 2 * c.n_kv_heads) * c.head_dim, nact = (size_t)R * c.trunk_inter;
+    const size_t nqkv = (size_t)LX_M * (c.n_q_heads + 2 * c.n_kv_heads) * c.head_dim, nact = (size_t)LX_M * c.trunk_inter;
     if (he == hipSuccess) he = dalloc(&e->lx_qkv, nqkv);
     if (he == hipSuccess) he = dalloc(&e->lx_act, nact);
     if (he == hipSuccess) he = hipMemset(e->lx_qkv, 0, nqkv * sizeof(uint2));
@@ -1279,7 +1284,7 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
     // all zero at creation: the first frame's first launch adds into
     // accumulator 1 (and a frame whose layer launches left early, after a
     // barrier timeout, still reads finite values)
-    if (he == hipSuccess) he = hipMemset(e->lx_acc, 0, 3 * (size_t)R * d * sizeof(unsigned long long));
+    if (he == hipSuccess) he = hipMemset(e->lx_acc, 0, 3 * (size_t)LX_M * d * sizeof(unsigned long long));
     if (he == hipSuccess) he = hipMemset(e->lx_flags, 0, (size_t)LX_XCDS * LX_FLAGS * sizeof(unsigned));
     if (he == hipSuccess) he = hipMemset(e->lx_err, 0, sizeof(unsigned));
   }
@@ -1609,7 +1614,7 @@ int sk_capture(sk_engine* e) {
   if (e->exec) return SK_OK;
   SK_HIP(hipStreamSynchronize(e->stream));
   e->code_tables = !e->wide && e->c.n_utts == 1 &&
-                   code_tables_fit(e->c.d_model, e->rows, e->c.depth_inner, e->c.audio_vocab, e->c.weight_dtype);
+                   code_tables_fit(e->c.d_model, e->rows, e->c.depth_inner, e->c.audio_vocab);
   e->wide_tables = e->wide && e->c.depth_inner <= SNT * DEPTH_API && e->c.d_model <= SNT * DEPTH_DPT;
   if ((e->code_tables || e->wide_tables) && (rc = build_code_tables(e)) != SK_OK) return rc;
   if (e->code_tables && e->prefilled) SK_HIP(launch_g1(e));   // a prefill before the capture did not compute G_1

@@ -2512,7 +2512,8 @@ __device__ __forceinline__ float2 rope_cs(int p, float fq) {
 }
 
 // ------------------------------------------------------------ depth step (code tables)
-// One utterance's depth step with the SwiGLU input taken apart by linearity.
+// One utterance's depth step (M = 2 rows with CFG, 1 without) with the SwiGLU
+// input taken apart by linearity.
 // The gate/up input of codebook q is a_q = w_in * x_q * r_q, with x_q = hidden +
 // prefix_q, r_q = 1 / rms(x_q), and x_q = x_{q-1} + scale * table[q-1][c] once
 // code c of codebook q-1 is drawn.  So
@@ -2533,8 +2534,8 @@ __device__ __forceinline__ float2 rope_cs(int p, float fq) {
 // Work of one launch (256 workgroups of SNT threads): for G_1 each wave owns
 // RWG gate rows and the same RWG up rows of W_gu (whole rows, K = KD); for the
 // down projection the workgroup owns RD = KD / 256 output rows while its 8
-// waves split the inner dimension KI into 8 chunks of 64 * VEC (one 16-byte
-// weight load per lane and row).  Every weight load is issued before the
+// waves split the inner dimension KI into 8 chunks of 64 * CV (a lane's CV
+// weights per row: 8 to 32 bytes).  Every weight load is issued before the
 // sampler runs.
 //   MODE 0: G_1 = W_gu (w_in * hidden) only (x_0 = hidden; no sampler).
 //   MODE 1: codebook 0's SwiGLU + down: act_0 = SwiGLU(r_0 G_1), y_0.
@@ -2572,6 +2573,30 @@ struct DepthArgs {
 };
 constexpr int DEPTH_WGS = 256;
 
+// N consecutive weights (8, 16 or 32 bytes) held as loaded, widened where used.
+template <typename TL, int N>
+struct RowPiece {
+  static constexpr int W = N * (int)sizeof(typename TL::elem) / 4;
+  uint32_t w[W];
+  __device__ __forceinline__ void load(const void* base, size_t off) {
+    const typename TL::elem* p = static_cast<const typename TL::elem*>(base) + off;
+    if constexpr (W == 2) {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      w[0] = v.x; w[1] = v.y;
+    } else {
+#pragma unroll
+      for (int i = 0; i < W; i += 4) {
+        const uint4 v = reinterpret_cast<const uint4*>(p)[i / 4];
+        w[i] = v.x; w[i + 1] = v.y; w[i + 2] = v.z; w[i + 3] = v.w;
+      }
+    }
+  }
+  __device__ __forceinline__ float get(int i) const {
+    if constexpr (sizeof(typename TL::elem) == 4) return __uint_as_float(w[i]);
+    else return __uint_as_float(i & 1 ? w[i / 2] & 0xffff0000u : w[i / 2] << 16);
+  }
+};
+
 template <typename TL, int VPT, int M, int KD, int KI, int MODE>
 __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs g, int q) {
   extern __shared__ unsigned char raw[];
@@ -2586,7 +2611,8 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
   constexpr int RWG = KI / (DEPTH_WGS * SWAVES);
   constexpr int RD = KD / DEPTH_WGS;
   static_assert(KD % (64 * VEC) == 0 && KD % SNT == 0 && KD % DEPTH_WGS == 0 && M <= 2, "depth_step shape");
-  static_assert(RWG >= 1 && RWG * DEPTH_WGS * SWAVES == KI && KI == SWAVES * 64 * VEC, "depth_step inner");
+  constexpr int CV = KI / (SWAVES * 64);        // inner indices per lane (its wave's chunk)
+  static_assert(RWG >= 1 && RWG * DEPTH_WGS * SWAVES == KI && CV * SWAVES * 64 == KI && CV % 4 == 0, "depth_step inner");
   __shared__ SampleSmem s;
   __shared__ __attribute__((aligned(16))) float xsh[M * KD];
   __shared__ __attribute__((aligned(16))) float gsh[KD];
@@ -2662,15 +2688,15 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
   // G_q at this lane's inner indices of its wave's chunk (gate and up): at
   // entry without a sampler, else with the code's table entries after it
   // (they are needed only then, and they do not hold registers through it).
-  const int kc = (wave * 64 + lane) * VEC;
-  float gq[M][2][VEC];
+  const int kc = (wave * 64 + lane) * CV;
+  float gq[M][2][CV];
   auto load_gq = [&]() {
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < VEC; i += 4) {
+        for (int i = 0; i < CV; i += 4) {
           const float4 t = *reinterpret_cast<const float4*>(g.g_in + (size_t)m * 2 * KI + h * KI + kc + i);
           gq[m][h][i] = t.x; gq[m][h][i + 1] = t.y; gq[m][h][i + 2] = t.z; gq[m][h][i + 3] = t.w;
         }
@@ -2697,10 +2723,10 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
   // for: at the 1.7B shape its 16.8 MB held them back ~1.6 us), so they
   // stream while the sampler runs.
   const int row0 = blockIdx.x * RD;
-  uint4 wd[DPART ? RD : 1];
+  RowPiece<TL, CV> wd[DPART ? RD : 1];
   if constexpr (DPART && !SAMPLE) {
 #pragma unroll
-    for (int i = 0; i < RD; ++i) wd[i] = TL::raw(g.w_down, (size_t)(row0 + i) * KI + kc);
+    for (int i = 0; i < RD; ++i) wd[i].load(g.w_down, (size_t)(row0 + i) * KI + kc);
   }
   __builtin_amdgcn_sched_barrier(0);
   // MODE 4, 5: the bookkeeping loads that depend on a position or the frame
@@ -2728,14 +2754,14 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
                            (lead && P.record_logits) ? a.dbg + (size_t)qs * a.V : nullptr, xr);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < RD; ++i) wd[i] = TL::raw(g.w_down, (size_t)(row0 + i) * KI + kc);
+    for (int i = 0; i < RD; ++i) wd[i].load(g.w_down, (size_t)(row0 + i) * KI + kc);
     __builtin_amdgcn_sched_barrier(0);
   }
 
   // The code of codebook q-1 (every workgroup draws the same one), then its
   // table row and its code-table entries at this lane's chunk.
   int code = 0;
-  float tv[DPT], pr[2][VEC];
+  float tv[DPT], pr[2][CV];
   if constexpr (SAMPLE) {
     const bool q0 = (qs == 0) && P.has_q0;
     code = sample_core<VPT>(xr, a.V, q0 ? P.temperature_q0 : P.temperature, q0 ? P.top_k_q0 : P.top_k,
@@ -2760,7 +2786,7 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < VEC; i += 4) {
+      for (int i = 0; i < CV; i += 4) {
         const float4 t = *reinterpret_cast<const float4*>(pp + h * KI + i);
         pr[h][i] = t.x; pr[h][i + 1] = t.y; pr[h][i + 2] = t.z; pr[h][i + 3] = t.w;
       }
@@ -2873,8 +2899,8 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
       }
     }
     // word (r * 2 + h) * M + m; its total lands in lanes word * (64 / NG) ...
-    constexpr int NG = RWG * 2 * M;
-    float wv[NG];
+    constexpr int NW = RWG * 2 * M, NG = NW < 4 ? 4 : NW;   // wave_reduce_words takes 4 words or more
+    float wv[NG] = {};
 #pragma unroll
     for (int r = 0; r < RWG; ++r)
 #pragma unroll
@@ -2882,7 +2908,7 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
 #pragma unroll
         for (int m = 0; m < M; ++m) wv[(r * 2 + h) * M + m] = acc[r][h][m];
     const float tot = wave_reduce_words<NG>(wv, lane);
-    if (lane % (64 / NG) == 0) {
+    if (lane % (64 / NG) == 0 && lane / (64 / NG) < NW) {
       const int word = lane / (64 / NG), m = word % M, h = (word / M) % 2, r = word / (2 * M);
       g.g_out[(size_t)m * 2 * KI + h * KI + n0 + r] = tot;
     }
@@ -2906,12 +2932,12 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
 
   // act = SwiGLU(r (G_q + scale P[c])) at this lane's chunk; y = a + W_d act
   if constexpr (DPART) {
-    float act[M][VEC];
-    float gnext[MODE == 2 ? M : 1][2][VEC];
+    float act[M][CV];
+    float gnext[MODE == 2 ? M : 1][2][CV];
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
-      for (int i = 0; i < VEC; ++i) {
+      for (int i = 0; i < CV; ++i) {
         float gt = gq[m][0][i], up = gq[m][1][i];
         if constexpr (SAMPLE) {
           gt = fmaf(g.scale, pr[0][i], gt);
@@ -2935,7 +2961,7 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
 #pragma unroll
           for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < VEC; i += 4)
+            for (int i = 0; i < CV; i += 4)
               *reinterpret_cast<float4*>(g.g_out + (size_t)m * 2 * KI + h * KI + kc + i) =
                   make_float4(gnext[m][h][i], gnext[m][h][i + 1], gnext[m][h][i + 2], gnext[m][h][i + 3]);
       }
@@ -2944,13 +2970,14 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
     float dw[ND];
 #pragma unroll
     for (int i = 0; i < RD; ++i) {
-      float w[VEC];
-      TL::widen(wd[i], w);
+      float w[CV];
+#pragma unroll
+      for (int e = 0; e < CV; ++e) w[e] = wd[i].get(e);
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         float t = 0.f;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) t = fmaf(w[e], act[m][e], t);
+        for (int e = 0; e < CV; ++e) t = fmaf(w[e], act[m][e], t);
         dw[i * M + m] = t;
       }
     }
@@ -2971,9 +2998,6 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
   }
 }
 
-__host__ __device__ constexpr bool depth_step_fits(int d, int inner, int vec) {
-  return (d == 1024 || d == 2048) && inner == SWAVES * 64 * vec && inner % (DEPTH_WGS * SWAVES) == 0;
-}
 
 // Code tables P_j[c] = W_gu (w_in * table[j][c]) are built with the prefill
 // GEMM from rows of table[j] times the norm gain (FP32).
