@@ -53,7 +53,7 @@ hipError_t dalloc(T** p, size_t n) {
 // O and down projections' slices (P) use QKV and Q, which are dead by then.
 struct PrefillBufs {
   float *X = nullptr, *Xn = nullptr, *QKV = nullptr, *Q = nullptr, *ATT = nullptr, *ACT = nullptr;
-  int *tok_row = nullptr, *tok_pos = nullptr;
+  int *tok_row = nullptr, *tok_pos = nullptr, *tok_src = nullptr;   // in the engine's pf_tab; the codes follow
   int qkv_split = 1, p_split = 1;   // most K slices that fit
 };
 
@@ -91,7 +91,7 @@ struct PrefillSizes { size_t qkv, total; };
 PrefillSizes prefill_sizes(const sk_config& c, int nqkv, size_t M) {
   const size_t hq = (size_t)c.n_q_heads * c.head_dim;
   const size_t rest = up256(M * c.d_model * 4) * 2 + up256(M * hq * 4) * 2 + up256(M * c.trunk_inter * 4) +
-                      up256(M * 4) * 2;
+                      up256(M * 4) * 2;   // (two token tables, now elsewhere: the size that fits stays what it was)
   const size_t one = up256(M * nqkv * 4), room = SK_NOALLOC_SCRATCH_BYTES;
   size_t qkv = std::max(one, std::min<size_t>(4u << 20, rest < room ? (room - rest) & ~(size_t)255 : 0));
   return PrefillSizes{qkv, rest + qkv};
@@ -110,8 +110,6 @@ PrefillBufs carve_prefill(const sk_config& c, int nqkv, size_t M, void* base) {
   b.Q = reinterpret_cast<float*>(take(M * hq * 4));
   b.ATT = reinterpret_cast<float*>(take(M * hq * 4));
   b.ACT = reinterpret_cast<float*>(take(M * c.trunk_inter * 4));
-  b.tok_row = reinterpret_cast<int*>(take(M * 4));
-  b.tok_pos = reinterpret_cast<int*>(take(M * 4));
   b.qkv_split = (int)std::min<size_t>(GEMM_MAX_SPLIT, z.qkv / (M * nqkv * 4));
   b.p_split = (int)std::max<size_t>(1, std::min<size_t>(GEMM_MAX_SPLIT, (z.qkv + M * hq * 4) / (M * c.d_model * 4)));
   return b;
@@ -144,7 +142,7 @@ struct sk_engine {
   float *qkv = nullptr, *attn = nullptr, *act = nullptr, *logits = nullptr;
   char *kc = nullptr, *vc = nullptr;   // KV caches, cfg.kv_dtype elements
   float *inv_freq = nullptr;
-  float *part = nullptr, *dbg = nullptr, *embeds = nullptr;
+  float *part = nullptr, *dbg = nullptr;
   float2* rope = nullptr;     // [rows][hd/2] (cos, sin) at each row's position
   float* sk_partial = nullptr;  // many-row path: split-K slice partials
   unsigned* sk_arrive = nullptr;
@@ -156,10 +154,14 @@ struct sk_engine {
   // their producers) and per-tile sums of squares for the RMSNorms.
   uint16_t *xs_x = nullptr, *xs_attn = nullptr, *xs_act = nullptr, *xs_abuf = nullptr, *xs_y = nullptr;
   float *ss_x = nullptr, *ss_y = nullptr;   // [32][d_model / 16]
-  int *kv_len = nullptr, *pos = nullptr, *active = nullptr, *plen = nullptr;
+  int *kv_len = nullptr, *pos = nullptr, *active = nullptr, *plen = nullptr;   // plen, p_row_start: in pf_tab
   int *fc = nullptr, *flag_ring = nullptr, *flag_cur = nullptr;
   double *u_ring = nullptr, *u_cur = nullptr;
-  int64_t *forced_ring = nullptr, *codes_ring = nullptr, *stage_ids = nullptr, *stage_codes = nullptr;
+  int64_t *forced_ring = nullptr, *codes_ring = nullptr;
+  // prefixes staged by sk_prefill_row, until the prefill runs: per row its text
+  // ids and the codes of its frames
+  std::vector<std::vector<int>> ids_host, frames_host;
+  int* pf_tab = nullptr;                   // the prefill's tables (prefill_staged), sized for every row full
   int* codes_cur = nullptr;
   SkParams* params = nullptr;
 
@@ -902,22 +904,19 @@ hipError_t ensure_prefill_bufs(sk_engine* e, int M) {
 }
 
 template <bool BF, int NCH>
-hipError_t launch_pf_norm_t(const sk_engine* e, bool first, int M, const PrefillBufs& b, int ns, size_t slice,
-                            const float* w) {
+hipError_t launch_pf_norm_t(const sk_engine* e, int M, const PrefillBufs& b, int ns, size_t slice, const float* w) {
   const sk_config& c = e->c;
-  hipLaunchKernelGGL((pf_norm_kernel<BF, NCH>), dim3(M), dim3(NT), 0, e->stream, first ? e->embeds : nullptr,
-                     c.max_ctx, b.tok_row, b.tok_pos, b.QKV, ns, slice, w, c.trunk_eps, c.d_model, b.X, b.Xn,
-                     reinterpret_cast<uint16_t*>(b.Xn), (size_t)M * c.d_model);
+  hipLaunchKernelGGL((pf_norm_kernel<BF, NCH>), dim3(M), dim3(NT), 0, e->stream, b.QKV, ns, slice, w,
+                     c.trunk_eps, c.d_model, b.X, b.Xn, reinterpret_cast<uint16_t*>(b.Xn), (size_t)M * c.d_model);
   return hipGetLastError();
 }
 template <bool BF>
-hipError_t launch_pf_norm(const sk_engine* e, bool first, int M, const PrefillBufs& b, int ns, size_t slice,
-                          const float* w) {
+hipError_t launch_pf_norm(const sk_engine* e, int M, const PrefillBufs& b, int ns, size_t slice, const float* w) {
   const int d = e->c.d_model;
-  if (d <= 4 * NT) return launch_pf_norm_t<BF, 1>(e, first, M, b, ns, slice, w);
-  if (d <= 8 * NT) return launch_pf_norm_t<BF, 2>(e, first, M, b, ns, slice, w);
-  if (d <= 16 * NT) return launch_pf_norm_t<BF, 4>(e, first, M, b, ns, slice, w);
-  return launch_pf_norm_t<BF, 0>(e, first, M, b, ns, slice, w);
+  if (d <= 4 * NT) return launch_pf_norm_t<BF, 1>(e, M, b, ns, slice, w);
+  if (d <= 8 * NT) return launch_pf_norm_t<BF, 2>(e, M, b, ns, slice, w);
+  if (d <= 16 * NT) return launch_pf_norm_t<BF, 4>(e, M, b, ns, slice, w);
+  return launch_pf_norm_t<BF, 0>(e, M, b, ns, slice, w);
 }
 
 template <typename KT, int HD, int WK, bool BF>
@@ -976,11 +975,15 @@ hipError_t enqueue_prefill_t(sk_engine* e, int M, int max_len, const PrefillBufs
     g.M = M; g.N = N; g.K = K; g.ksplit = p.ksplit;
     return g;
   };
+  hipLaunchKernelGGL((pf_embed_kernel<typename std::conditional<BF, WBF16, WF32>::type>), dim3(M), dim3(NT), 0, st,
+                     b.tok_src, b.tok_src + M, e->embed_tokens, e->lang, c.n_language, c.language_ids[0],
+                     c.language_ids[1], c.language_ids[2], c.language_ids[3], e->table, c.n_codebooks, c.audio_vocab,
+                     d, c.frame_scale, b.X);
   for (int l = 0; l < c.n_layers; ++l) {
     const LayerW& w = e->L[l];
     KT* kc = reinterpret_cast<KT*>(e->kc + (size_t)l * kv_layer_bytes(e));
     KT* vc = reinterpret_cast<KT*>(e->vc + (size_t)l * kv_layer_bytes(e));
-    if ((err = launch_pf_norm<BF>(e, l == 0, M, b, l == 0 ? 0 : nd, pslice, w.in_norm)) != hipSuccess) return err;
+    if ((err = launch_pf_norm<BF>(e, M, b, l == 0 ? 0 : nd, pslice, w.in_norm)) != hipSuccess) return err;
     GemmArgs g = gemm(pq, b.Xn, w.q, e->nqkv, d, b.QKV);
     g.B[1] = w.k; g.B[2] = w.v;
     g.seg_rows[0] = hq; g.seg_rows[1] = c.n_kv_heads * hd; g.seg_rows[2] = c.n_kv_heads * hd;
@@ -993,7 +996,7 @@ hipError_t enqueue_prefill_t(sk_engine* e, int M, int max_len, const PrefillBufs
     g = gemm(po, b.ATT, w.o, d, hq, no ? b.QKV : b.X);
     g.res = no ? nullptr : b.X;
     if ((err = launch_gemm<GEPI_STORE>(BF, po.tile, g, st)) != hipSuccess) return err;
-    if ((err = launch_pf_norm<BF>(e, false, M, b, no, pslice, w.post_norm)) != hipSuccess) return err;
+    if ((err = launch_pf_norm<BF>(e, M, b, no, pslice, w.post_norm)) != hipSuccess) return err;
     g = gemm(pg, b.Xn, w.gate, I, d, b.ACT);
     g.B2 = w.up;
     g.xs = reinterpret_cast<uint16_t*>(b.ACT); g.xs_lo = (size_t)M * I;
@@ -1152,6 +1155,8 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
   e->active_host.assign(e->rows, 0);
   e->len_host.assign(e->rows, 0);
   e->staged.assign(e->rows, 0);
+  e->ids_host.resize(e->rows);
+  e->frames_host.resize(e->rows);
   auto bail = [&](int code) { sk_destroy(e); return code; };
 #define ALLOC(ptr, n)                                                                   \
   do {                                                                                  \
@@ -1207,10 +1212,9 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
     ALLOC(e->xs_act, xsplit_elems(e->inner_max)); ALLOC(e->xs_abuf, xsplit_elems(d)); ALLOC(e->xs_y, xsplit_elems(d));
     ALLOC(e->ss_x, (size_t)XS_ROWS * d / 16); ALLOC(e->ss_y, (size_t)XS_ROWS * d / 16);
   }
-  ALLOC(e->kv_len, RA); ALLOC(e->pos, RA); ALLOC(e->active, RA); ALLOC(e->plen, R);
+  ALLOC(e->kv_len, RA); ALLOC(e->pos, RA); ALLOC(e->active, RA);
   ALLOC(e->fc, 1);
   ALLOC(e->p_rope, (size_t)(c.max_ctx + 1) * (c.head_dim / 2));
-  ALLOC(e->p_row_start, R);
   ALLOC(e->u_ring, (size_t)c.max_frames * c.n_utts * Q);
   ALLOC(e->flag_ring, (size_t)c.max_frames * 2);
   ALLOC(e->u_cur, (size_t)c.n_utts * Q);
@@ -1219,9 +1223,7 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
   ALLOC(e->forced_ring, (size_t)c.max_frames * c.n_utts * Q);
   ALLOC(e->codes_ring, (size_t)c.max_frames * c.n_utts * Q);
   ALLOC(e->dbg, (size_t)c.n_utts * Q * V);
-  ALLOC(e->embeds, R * c.max_ctx * d);
-  ALLOC(e->stage_ids, (size_t)c.max_ctx);
-  ALLOC(e->stage_codes, (size_t)c.max_ctx * Q);
+  ALLOC(e->pf_tab, 2 * R + R * c.max_ctx * (3 + Q));
   ALLOC(e->params, 1);
 #undef ALLOC
   const std::vector<float> inv = rope_inv_freq(c);
@@ -1304,13 +1306,13 @@ int sk_destroy(sk_engine* e) {
   if (e->stream) hipStreamSynchronize(e->stream);
   drop_graphs(e);
   void* bufs[] = {e->sk_partial, e->sk_arrive, e->sk_tpart, e->sk_err, e->xs_x, e->xs_attn, e->xs_act, e->xs_abuf, e->xs_y, e->ss_x, e->ss_y, e->x, e->hidden, e->prefix, e->prefix2, e->abuf, e->ybuf, e->qkv, e->attn, e->act, e->logits,
-                  e->kc, e->vc, e->inv_freq, e->rope, e->part, e->dbg, e->embeds, e->u_cur, e->flag_cur, e->codes_cur,
-                  e->kv_len, e->pos, e->active, e->plen, e->fc, e->flag_ring, e->u_ring,
+                  e->kc, e->vc, e->inv_freq, e->rope, e->part, e->dbg, e->pf_tab, e->u_cur, e->flag_cur, e->codes_cur,
+                  e->kv_len, e->pos, e->active, e->fc, e->flag_ring, e->u_ring,
                   e->pf_mem, e->ptab, e->gbuf[0], e->gbuf[1],
                   e->lx_acc, e->lx_qkv, e->lx_act,
                   e->lx_flags, e->lx_err,
-                  e->p_row_start, e->p_rope,
-                  e->forced_ring, e->codes_ring, e->stage_ids, e->stage_codes, e->params};
+                  e->p_rope,
+                  e->forced_ring, e->codes_ring, e->params};
   for (void* p : bufs)
     if (p) hipFree(p);
   if (e->order_ev) hipEventDestroy(e->order_ev);
@@ -1396,24 +1398,10 @@ int sk_prefill_row(sk_engine* e, int32_t row, const int64_t* text_ids, int32_t n
   SK_CHECK(n_text == 0 || e->embed_tokens, SK_ENOWEIGHT, "trunk.embed_tokens.weight is not bound");
   SK_CHECK(n_frames == 0 || e->table, SK_ENOWEIGHT, "audio_codebooks.table is not bound");
   SK_CHECK(c.n_language == 0 || n_text == 0 || e->lang, SK_ENOWEIGHT, "language_embeddings.weight is not bound");
-  if (n_text) SK_HIP(hipMemcpyAsync(e->stage_ids, text_ids, n_text * sizeof(int64_t), hipMemcpyHostToDevice, e->stream));
-  if (n_frames)
-    SK_HIP(hipMemcpyAsync(e->stage_codes, frame_codes, (size_t)n_frames * c.n_codebooks * sizeof(int64_t),
-                          hipMemcpyHostToDevice, e->stream));
-  float* dst = e->embeds + (size_t)row * c.max_ctx * c.d_model;
+  // Only kept here: the prefill embeds every staged row's tokens in one launch.
   const int n = n_text + n_frames;
-  if (c.weight_dtype == SK_BF16)
-    hipLaunchKernelGGL(embed_prefix_kernel<WBF16>, dim3(n), dim3(NT), 0, e->stream, e->stage_ids, n_text,
-                       e->stage_codes, e->embed_tokens, e->lang, c.n_language, c.language_ids[0],
-                       c.language_ids[1], c.language_ids[2], c.language_ids[3], e->table, c.n_codebooks,
-                       c.audio_vocab, c.d_model, c.frame_scale, dst);
-  else
-    hipLaunchKernelGGL(embed_prefix_kernel<WF32>, dim3(n), dim3(NT), 0, e->stream, e->stage_ids, n_text,
-                       e->stage_codes, e->embed_tokens, e->lang, c.n_language, c.language_ids[0],
-                       c.language_ids[1], c.language_ids[2], c.language_ids[3], e->table, c.n_codebooks,
-                       c.audio_vocab, c.d_model, c.frame_scale, dst);
-  SK_HIP(hipGetLastError());
-  SK_HIP(hipStreamSynchronize(e->stream));
+  e->ids_host[row].assign(text_ids, text_ids + n_text);
+  e->frames_host[row].assign(frame_codes, frame_codes + (size_t)n_frames * c.n_codebooks);
   e->len_host[row] = n;
   e->staged[row] = 1;
   e->prefilled = false;
@@ -1444,15 +1432,29 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
   SK_CHECK(n_staged > 0, SK_ESTATE, "no row has a staged prefix");
   int rc = check_decode_weights(e);
   if (rc != SK_OK) return rc;
-  // Pack the staged rows' prefix tokens row after row.
-  std::vector<int> row_start(R), row_len(R), tok_row, tok_pos;
+  // Pack the staged rows' prefix tokens row after row, in one table of ints:
+  // row lengths, row starts, then per token its row, its position and its
+  // source (text id, or -1 - frame), then the frames' codes.
   int M = 0, max_len = 0;
+  size_t n_codes = 0;
+  for (int r = 0; r < R; ++r)
+    if (e->staged[r]) { M += e->len_host[r]; n_codes += e->frames_host[r].size(); }
+  std::vector<int> tab(2 * (size_t)R + 3 * (size_t)M + n_codes);
+  int* row_len = tab.data();
+  int *row_start = row_len + R, *tok_row = row_start + R, *tok_pos = tok_row + M, *tok_src = tok_pos + M;
+  int* codes = tok_src + M;
+  int m = 0, nf = 0;
   for (int r = 0; r < R; ++r) {
-    row_start[r] = M;
+    row_start[r] = m;
     row_len[r] = e->staged[r] ? e->len_host[r] : 0;
-    for (int p = 0; p < row_len[r]; ++p) { tok_row.push_back(r); tok_pos.push_back(p); }
-    M += row_len[r];
-    max_len = row_len[r] > max_len ? row_len[r] : max_len;
+    const int nt = (int)e->ids_host[r].size();
+    for (int p = 0; p < row_len[r]; ++p, ++m) {
+      tok_row[m] = r;
+      tok_pos[m] = p;
+      tok_src[m] = p < nt ? e->ids_host[r][p] : -1 - nf++;
+    }
+    if (row_len[r]) codes = std::copy(e->frames_host[r].begin(), e->frames_host[r].end(), codes);
+    max_len = std::max(max_len, row_len[r]);
   }
   PrefillBufs bufs;
   if (noalloc) {
@@ -1474,10 +1476,12 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
     // the no-alloc scratch) take turns
     std::lock_guard<std::mutex> lk(g_frame_order[e->device].mu);
     SK_HIP(order_after_previous(e));
-    SK_HIP(hipMemcpyAsync(e->plen, row_len.data(), R * sizeof(int), hipMemcpyHostToDevice, e->stream));
-    SK_HIP(hipMemcpyAsync(e->p_row_start, row_start.data(), R * sizeof(int), hipMemcpyHostToDevice, e->stream));
-    SK_HIP(hipMemcpyAsync(bufs.tok_row, tok_row.data(), M * sizeof(int), hipMemcpyHostToDevice, e->stream));
-    SK_HIP(hipMemcpyAsync(bufs.tok_pos, tok_pos.data(), M * sizeof(int), hipMemcpyHostToDevice, e->stream));
+    e->plen = e->pf_tab;
+    e->p_row_start = e->plen + R;
+    bufs.tok_row = e->p_row_start + R;
+    bufs.tok_pos = bufs.tok_row + M;
+    bufs.tok_src = bufs.tok_pos + M;
+    SK_HIP(hipMemcpyAsync(e->pf_tab, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice, e->stream));
     if (all) {
       SK_HIP(hipMemsetAsync(e->fc, 0, sizeof(int), e->stream));
       SK_HIP(clear_split_tags(e));

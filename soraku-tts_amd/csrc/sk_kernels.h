@@ -3256,36 +3256,6 @@ __global__ __launch_bounds__(NT) void final_norm_kernel(const float* x, const lo
   }
 }
 
-// Prefix embeddings of one row: text rows (language rows replaced,
-// model.py:326-338), then frame embeddings (model.py:105-114).
-template <typename TL>
-__global__ __launch_bounds__(NT) void embed_prefix_kernel(const int64_t* ids, int n_text,
-                                                          const int64_t* codes, const void* embed,
-                                                          const float* lang_table, int n_lang,
-                                                          int l0, int l1, int l2, int l3,
-                                                          const void* table, int Q, int V, int D,
-                                                          float scale, float* out) {
-  const int i = blockIdx.x;
-  float* o = out + (size_t)i * D;
-  if (i < n_text) {
-    const int64_t id = ids[i];
-    int lj = -1;
-    if (n_lang > 0) lj = (id == l0) ? 0 : (id == l1) ? 1 : (id == l2) ? 2 : (id == l3) ? 3 : -1;
-    for (int k = threadIdx.x; k < D; k += NT)
-      o[k] = (lj >= 0) ? lang_table[(size_t)lj * D + k] : TL::get(embed, (size_t)id * D + k);
-  } else {
-    const int64_t* c = codes + (size_t)(i - n_text) * Q;
-    for (int k = threadIdx.x; k < D; k += NT) {
-      float e = 0.f;
-      for (int j = 0; j < Q; ++j) {
-        const float t = TL::get(table, ((size_t)j * V + (size_t)c[j]) * D + k);
-        e = (j == 0) ? t : __fadd_rn(e, t);
-      }
-      o[k] = __fmul_rn(e, scale);
-    }
-  }
-}
-
 // ---- operator-API elementwise kernels (tilelang_kernels.py:176-254) ----
 __global__ __launch_bounds__(NT) void frame_embed_op_kernel(const int64_t* codes, const float* table,
                                                             int Q, int V, int D, float scale,

@@ -3,7 +3,7 @@
 // modeling_qwen3.py:367-427).  Tokens are packed row after row: token m is
 // row tok_row[m] at position tok_pos[m]; row r's tokens start at row_start[r].
 //
-//   X = embeds -> per layer: Xn = RMSNorm(X); QKV = Xn Wqkv^T (MFMA GEMM,
+//   X = prefix embeddings -> per layer: Xn = RMSNorm(X); QKV = Xn Wqkv^T (MFMA GEMM,
 //   sk_gemm.h); QK-norm + RoPE, K/V written into the decode cache; causal
 //   attention per row; P = Att Wo^T; X += P, Xn = RMSNorm(X); Act = silu(Xn
 //   Wg^T) * (Xn Wu^T); P = Act Wd^T, added to X by the next norm -> hidden =
@@ -20,29 +20,73 @@
 
 namespace sk {
 
+// ------------------------------------------------------------ prefix embeddings
+// X[m] for every packed token: src[m] >= 0 a text id (language rows replaced,
+// model.py:326-338), else frame -1 - src[m] of codes [frames][Q]: scale *
+// sum_q table[q, code q], in q order (model.py:105-114).  One launch for all
+// rows, 8 table rows in flight per thread; each row used to be embedded by a
+// launch of its own (20-60 us: its 16 table rows one after another), copied in
+// and waited for when it was staged.
+template <typename TL>
+__global__ __launch_bounds__(NT) void pf_embed_kernel(const int* src, const int* codes, const void* embed,
+                                                      const float* lang_table, int n_lang, int l0, int l1, int l2,
+                                                      int l3, const void* table, int Q, int V, int D, float scale,
+                                                      float* X) {
+  const int m = blockIdx.x, id = src[m];
+  for (int k = threadIdx.x * 4; k < D; k += NT * 4) {
+    float e[4];
+    if (id >= 0) {
+      const int lj = n_lang == 0 ? -1 : id == l0 ? 0 : id == l1 ? 1 : id == l2 ? 2 : id == l3 ? 3 : -1;
+      if (lj >= 0) {
+        const float4 t = *reinterpret_cast<const float4*>(lang_table + (size_t)lj * D + k);
+        e[0] = t.x; e[1] = t.y; e[2] = t.z; e[3] = t.w;
+      } else {
+        RowPiece<TL, 4> t;
+        t.load(embed, (size_t)id * D + k);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = t.get(i);
+      }
+    } else {
+      const int* c = codes + (size_t)(-1 - id) * Q;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = 0.f;
+      for (int j0 = 0; j0 < Q; j0 += 8) {
+        RowPiece<TL, 4> t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int q = min(j0 + j, Q - 1);
+          t[j].load(table, ((size_t)q * V + c[q]) * D + k);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (j0 + j < Q) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) e[i] = j0 + j == 0 ? t[j].get(i) : __fadd_rn(e[i], t[j].get(i));
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = __fmul_rn(e[i], scale);
+    }
+    *reinterpret_cast<float4*>(X + (size_t)m * D + k) = make_float4(e[0], e[1], e[2], e[3]);
+  }
+}
+
 // ------------------------------------------------------------ residual + norm
-// Token m: x = residual + the ns K slices of the GEMM before it (P, in slice
-// order; ns = 0: that GEMM added to X itself), written back to X; Xn =
+// Token m: x = residual X[m] + the ns K slices of the GEMM before it (P, in
+// slice order; ns = 0: that GEMM added to X itself), written back to X; Xn =
 // RMSNorm(x) in the form the next GEMM takes (FP32, or BF16 hi / lo planes).
 // The slices' sum lives here because this kernel reads x anyway: a GEMM cut
-// into slices costs no launch of its own.  The residual is X[m], or for the
-// first layer (embeds != null) the prefix embedding of the token.  NCH: float4
-// of the row per thread, kept in registers (0: any D, the row is read back for
-// the norm).
+// into slices costs no launch of its own.  NCH: float4 of the row per thread,
+// kept in registers (0: any D, the row is read back for the norm).
 template <bool BF, int NCH>
-__global__ __launch_bounds__(NT) void pf_norm_kernel(const float* embeds, int max_ctx, const int* tok_row,
-                                                     const int* tok_pos, const float* P, int ns, size_t slice,
-                                                     const float* w, float eps, int D, float* X, float* Xn,
-                                                     uint16_t* xs, size_t xs_lo) {
+__global__ __launch_bounds__(NT) void pf_norm_kernel(const float* P, int ns, size_t slice, const float* w, float eps,
+                                                     int D, float* X, float* Xn, uint16_t* xs, size_t xs_lo) {
   __shared__ float red[WAVES];
   const int m = blockIdx.x, tid = threadIdx.x, D4 = D / 4;
-  const float4* src = reinterpret_cast<const float4*>(
-      embeds ? embeds + ((size_t)tok_row[m] * max_ctx + tok_pos[m]) * D : X + (size_t)m * D);
   const float4* pp = reinterpret_cast<const float4*>(P) + (size_t)m * D4;
   float4* xo = reinterpret_cast<float4*>(X) + (size_t)m * D4;
-  const bool keep = ns > 0 || embeds;        // x differs from X[m]
   auto load = [&](int k) {
-    float4 x = src[k];
+    float4 x = xo[k];
     float4 p[4];
     for (int s0 = 0; s0 < ns; s0 += 4) {
 #pragma unroll
@@ -74,7 +118,7 @@ __global__ __launch_bounds__(NT) void pf_norm_kernel(const float* embeds, int ma
       const int k = tid + c * NT;
       x[c] = load(min(k, D4 - 1));
       if (k < D4) {
-        if (keep) xo[k] = x[c];
+        if (ns) xo[k] = x[c];
         s += x[c].x * x[c].x + x[c].y * x[c].y + x[c].z * x[c].z + x[c].w * x[c].w;
       }
     }
@@ -85,7 +129,7 @@ __global__ __launch_bounds__(NT) void pf_norm_kernel(const float* embeds, int ma
   } else {
     for (int k = tid; k < D4; k += NT) {
       const float4 x = load(k);
-      if (keep) xo[k] = x;
+      if (ns) xo[k] = x;
       s += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
     }
     const float inv = 1.0f / sqrtf(block_sum(s, red) / (float)D + eps);
