@@ -165,6 +165,11 @@ struct sk_engine {
   int* codes_cur = nullptr;
   SkParams* params = nullptr;
 
+  // sk_step_frame's inputs and outputs in pinned host memory (frame_in_kernel,
+  // frame_out_kernel) and the device's addresses of them
+  double *pin_in = nullptr, *pin_in_dev = nullptr;
+  int64_t *pin_out = nullptr, *pin_out_dev = nullptr;
+
   // host mirrors
   int fc_host = 0;
   std::vector<int> active_host;   // rows decoding (advance each frame); retired rows do not
@@ -1226,6 +1231,18 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
   ALLOC(e->pf_tab, 2 * R + R * c.max_ctx * (3 + Q));
   ALLOC(e->params, 1);
 #undef ALLOC
+  {
+    const size_t nq = (size_t)c.n_utts * Q;
+    hipError_t pe = hipHostMalloc(reinterpret_cast<void**>(&e->pin_in), (2 * nq + 1) * sizeof(double), hipHostMallocCoherent);
+    if (pe == hipSuccess)
+      pe = hipHostMalloc(reinterpret_cast<void**>(&e->pin_out), (nq + 1) * sizeof(int64_t), hipHostMallocCoherent);
+    if (pe == hipSuccess) pe = hipHostGetDevicePointer(reinterpret_cast<void**>(&e->pin_in_dev), e->pin_in, 0);
+    if (pe == hipSuccess) pe = hipHostGetDevicePointer(reinterpret_cast<void**>(&e->pin_out_dev), e->pin_out, 0);
+    if (pe != hipSuccess) {
+      fail(SK_EHIP, "pinned frame buffers: %s", hipGetErrorString(pe));
+      return bail(SK_EHIP);
+    }
+  }
   const std::vector<float> inv = rope_inv_freq(c);
   hipError_t he = hipMemcpy(e->inv_freq, inv.data(), inv.size() * sizeof(float), hipMemcpyHostToDevice);
   if (he == hipSuccess) he = hipMemset(e->u_cur, 0, (size_t)c.n_utts * Q * sizeof(double));
@@ -1315,6 +1332,8 @@ int sk_destroy(sk_engine* e) {
                   e->forced_ring, e->codes_ring, e->params};
   for (void* p : bufs)
     if (p) hipFree(p);
+  if (e->pin_in) hipHostFree(e->pin_in);
+  if (e->pin_out) hipHostFree(e->pin_out);
   if (e->order_ev) hipEventDestroy(e->order_ev);
   if (e->stream) hipStreamDestroy(e->stream);
   delete e;
@@ -1636,17 +1655,17 @@ int sk_capture(sk_engine* e) {
   return SK_OK;
 }
 
-// The XCD-resident layers' error word (read after the stream is drained).
-static int check_lx(sk_engine* e) {
-  unsigned w = 0;
-  if (e->sk_err) {
-    SK_HIP(hipMemcpy(&w, e->sk_err, sizeof(w), hipMemcpyDeviceToHost));
-    SK_CHECK(w == 0u, SK_EHIP, "split-K merge wait timed out (error word 0x%x); the engine must be recreated", w);
-  }
-  if (!e->lx) return SK_OK;
-  SK_HIP(hipMemcpy(&w, e->lx_err, sizeof(w), hipMemcpyDeviceToHost));
-  SK_CHECK(w == 0u, SK_EHIP, "trunk layer barrier timed out (error word 0x%x); the engine must be recreated", w);
+// The engine's error words, as read after the stream is drained.
+static int check_err_words(unsigned split, unsigned layers) {
+  SK_CHECK(split == 0u, SK_EHIP, "split-K merge wait timed out (error word 0x%x); the engine must be recreated", split);
+  SK_CHECK(layers == 0u, SK_EHIP, "trunk layer barrier timed out (error word 0x%x); the engine must be recreated", layers);
   return SK_OK;
+}
+static int check_lx(sk_engine* e) {
+  unsigned w[2] = {0, 0};
+  if (e->sk_err) SK_HIP(hipMemcpy(&w[0], e->sk_err, sizeof(unsigned), hipMemcpyDeviceToHost));
+  if (e->lx) SK_HIP(hipMemcpy(&w[1], e->lx_err, sizeof(unsigned), hipMemcpyDeviceToHost));
+  return check_err_words(w[0], w[1]);
 }
 
 static int check_step(sk_engine* e, int n) {
@@ -1676,29 +1695,34 @@ int sk_step_frame(sk_engine* e, int32_t mask_eos_q0, const double* uniforms,
     for (size_t i = 0; i < nq; ++i)
       SK_CHECK(forced_codes[i] >= 0 && forced_codes[i] < c.audio_vocab, SK_EINVAL, "forced code out of range");
   const int slot = e->fc_host;
-  std::vector<double> u(nq, 0.0);
-  if (uniforms) memcpy(u.data(), uniforms, nq * sizeof(double));
+  // every earlier step has synchronised, so the pinned buffers are free
+  double* in = e->pin_in;
+  if (uniforms) memcpy(in, uniforms, nq * sizeof(double));
+  else std::fill(in, in + nq, 0.0);
   const int flags[2] = {mask_eos_q0, forced_codes ? 1 : 0};
-  SK_HIP(hipMemcpyAsync(e->u_ring + slot * nq, u.data(), nq * sizeof(double), hipMemcpyHostToDevice, e->stream));
-  SK_HIP(hipMemcpyAsync(e->flag_ring + 2 * slot, flags, sizeof(flags), hipMemcpyHostToDevice, e->stream));
-  SK_HIP(hipMemcpyAsync(e->u_cur, u.data(), nq * sizeof(double), hipMemcpyHostToDevice, e->stream));
-  SK_HIP(hipMemcpyAsync(e->flag_cur, flags, sizeof(flags), hipMemcpyHostToDevice, e->stream));
-  if (forced_codes)
-    SK_HIP(hipMemcpyAsync(e->forced_ring + slot * nq, forced_codes, nq * sizeof(int64_t), hipMemcpyHostToDevice,
-                          e->stream));
+  memcpy(in + nq, flags, sizeof(flags));
+  if (forced_codes) memcpy(in + nq + 1, forced_codes, nq * sizeof(int64_t));
   {
     std::lock_guard<std::mutex> lk(g_frame_order[e->device].mu);
     SK_HIP(order_after_previous(e));
+    hipLaunchKernelGGL(frame_in_kernel, dim3(1), dim3(NT), 0, e->stream, e->pin_in_dev, (int)nq, forced_codes != nullptr,
+                       e->u_ring + slot * nq, e->u_cur, e->flag_ring + 2 * slot, e->flag_cur, e->forced_ring + slot * nq);
+    SK_HIP(hipGetLastError());
     SK_HIP(set_frame_chunks(e, 0));
     SK_HIP(hipGraphLaunch(e->exec, e->stream));
+    hipLaunchKernelGGL(frame_out_kernel, dim3(1), dim3(NT), 0, e->stream, e->codes_ring + slot * nq, (int)nq, e->sk_err,
+                       e->lx ? e->lx_err : nullptr, e->pin_out_dev);
+    SK_HIP(hipGetLastError());
   }
-  SK_HIP(hipMemcpyAsync(codes_out, e->codes_ring + slot * nq, nq * sizeof(int64_t), hipMemcpyDeviceToHost, e->stream));
   if (logits_dbg)
     SK_HIP(hipMemcpyAsync(logits_dbg, e->dbg, nq * c.audio_vocab * sizeof(float), hipMemcpyDeviceToHost, e->stream));
   SK_HIP(hipStreamSynchronize(e->stream));
+  memcpy(codes_out, e->pin_out, nq * sizeof(int64_t));
   e->fc_host += 1;
   for (int r = 0; r < e->rows; ++r) e->kv_host[r] += e->active_host[r];
-  return check_lx(e);
+  unsigned w[2];
+  memcpy(w, e->pin_out + nq, sizeof(w));
+  return check_err_words(w[0], w[1]);
 }
 
 int sk_queue_frames(sk_engine* e, int32_t n, const double* uniforms, const int32_t* mask_eos_q0) {
