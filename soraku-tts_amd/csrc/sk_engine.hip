@@ -1149,11 +1149,21 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
   e->nqkv = (c.n_q_heads + 2 * c.n_kv_heads) * c.head_dim;
   e->inner_max = c.trunk_inter > c.depth_inner ? c.trunk_inter : c.depth_inner;
   e->max_chunks = (c.max_ctx + ATT_CHUNK - 1) / ATT_CHUNK;
-  // Many rows: streaming attention with enough splits per (row, kv head) for
-  // ~256 workgroups (one per CU); its partials reuse the chunk-partial buffer.
+  // Many rows: streaming attention, as many splits per (row, kv head) as fit
+  // the 256 CUs at one workgroup each (more leaves a second, nearly empty
+  // round); its partials reuse the chunk-partial buffer.  No split where a
+  // full row of the cache is at most 256 KB per head: reading that with one
+  // CU is cheaper than the merge launch and the partials.  us per frame,
+  // 0.6B, (splits: time), contexts half to all of the length stated:
+  //   6 rows FP32, 240 1: 1662, 5: 1684, 6: 1825; 480 1: 1780, 5: 1724; 960 1: 2018, 5: 1806, 6: 1990
+  //   8 rows FP32, 120 1: 1601, 4: 1692; 400 1: 1756, 4: 1722
+  //   8 rows BF16 (cache too), 400 1: 1389, 4: 1408; 800 1: 1515, 4: 1437
+  //   12 rows BF16, 240 1: 1350, 2: 1430, 3: 1592; 960 1: 1591, 2: 1547, 3: 1721
+  //   20 rows FP32, 400 1: 2057, 2: 2294; 1600 1: 2879, 2: 2963
   if (e->wide && (e->G == 1 || e->G == 2 || e->G == 4) && e->G * c.head_dim <= ATTN_STREAM_NTH) {
     const int pairs = e->rows * c.n_kv_heads;
-    e->attn_splits = std::max(1, std::min(e->max_chunks, (256 + pairs - 1) / pairs));
+    const size_t head_bytes = 2 * (size_t)c.max_ctx * c.head_dim * (c.kv_dtype == SK_BF16 ? 2 : 4);
+    e->attn_splits = head_bytes <= 256 * 1024 ? 1 : std::max(1, std::min(e->max_chunks, 256 / pairs));
   }
   e->L.resize(c.n_layers);
   e->kv_host.assign(e->rows, 0);
