@@ -63,13 +63,17 @@ struct GemmArgs {
 };
 
 // 16 bytes per lane from g straight into LDS at l + 16 * lane (l wave-uniform).
-// Written as assembly (M0 = the LDS address, which nothing else here uses) because with the builtin the compiler waits for every
+// Written as assembly because with the builtin the compiler waits for every
 // load in flight (vmcnt(0)) before the next LDS read, whichever part of the
-// ring it reads; the loop below does the waiting itself (wait_vm).  The
-// statement has no outputs: nothing is written but LDS.
+// ring it reads; the loop below does the waiting itself (stage_sync).  M0 holds
+// the LDS address and is declared overwritten: a value that the compiler keeps
+// there is set again afterwards (it does so, although it warns that M0 is a
+// reserved register).  The statement has no outputs: nothing is
+// written but LDS.
 __device__ __forceinline__ void lds_load16(const char* base, unsigned voff, const char* l) {
   const unsigned a = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)l);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(a) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(a)
+               : "memory", "m0");
 }
 
 // This wave's stage loads but the last N are in and its LDS reads are done;
