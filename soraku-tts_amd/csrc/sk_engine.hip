@@ -1690,6 +1690,28 @@ static int check_step(sk_engine* e, int n) {
   return SK_OK;
 }
 
+// A stepped frame's launches: inputs from the pinned buffer, the frame graph,
+// outputs to the pinned buffer (and the recorded logits to the host).
+static int enqueue_step(sk_engine* e, bool forced, float* logits_dbg) {
+  const size_t nq = (size_t)e->c.n_utts * e->c.n_codebooks;
+  const int slot = e->fc_host;
+  {
+    std::lock_guard<std::mutex> lk(g_frame_order[e->device].mu);
+    SK_HIP(order_after_previous(e));
+    hipLaunchKernelGGL(frame_in_kernel, dim3(1), dim3(NT), 0, e->stream, e->pin_in_dev, (int)nq, forced,
+                       e->u_ring + slot * nq, e->u_cur, e->flag_ring + 2 * slot, e->flag_cur, e->forced_ring + slot * nq);
+    SK_HIP(hipGetLastError());
+    SK_HIP(set_frame_chunks(e, 0));
+    SK_HIP(hipGraphLaunch(e->exec, e->stream));
+    hipLaunchKernelGGL(frame_out_kernel, dim3(1), dim3(NT), 0, e->stream, e->codes_ring + slot * nq, (int)nq, e->sk_err,
+                       e->lx ? e->lx_err : nullptr, e->pin_out_dev);
+    SK_HIP(hipGetLastError());
+  }
+  if (logits_dbg)
+    SK_HIP(hipMemcpyAsync(logits_dbg, e->dbg, nq * e->c.audio_vocab * sizeof(float), hipMemcpyDeviceToHost, e->stream));
+  return SK_OK;
+}
+
 int sk_step_frame(sk_engine* e, int32_t mask_eos_q0, const double* uniforms,
                   const int64_t* forced_codes, int64_t* codes_out, float* logits_dbg) {
   int rc = check_step(e, 1);
@@ -1704,28 +1726,17 @@ int sk_step_frame(sk_engine* e, int32_t mask_eos_q0, const double* uniforms,
   if (forced_codes)
     for (size_t i = 0; i < nq; ++i)
       SK_CHECK(forced_codes[i] >= 0 && forced_codes[i] < c.audio_vocab, SK_EINVAL, "forced code out of range");
-  const int slot = e->fc_host;
-  // every earlier step has synchronised, so the pinned buffers are free
+  // every earlier step has waited for its stream, so the pinned buffers are free
   double* in = e->pin_in;
   if (uniforms) memcpy(in, uniforms, nq * sizeof(double));
   else std::fill(in, in + nq, 0.0);
   const int flags[2] = {mask_eos_q0, forced_codes ? 1 : 0};
   memcpy(in + nq, flags, sizeof(flags));
   if (forced_codes) memcpy(in + nq + 1, forced_codes, nq * sizeof(int64_t));
-  {
-    std::lock_guard<std::mutex> lk(g_frame_order[e->device].mu);
-    SK_HIP(order_after_previous(e));
-    hipLaunchKernelGGL(frame_in_kernel, dim3(1), dim3(NT), 0, e->stream, e->pin_in_dev, (int)nq, forced_codes != nullptr,
-                       e->u_ring + slot * nq, e->u_cur, e->flag_ring + 2 * slot, e->flag_cur, e->forced_ring + slot * nq);
-    SK_HIP(hipGetLastError());
-    SK_HIP(set_frame_chunks(e, 0));
-    SK_HIP(hipGraphLaunch(e->exec, e->stream));
-    hipLaunchKernelGGL(frame_out_kernel, dim3(1), dim3(NT), 0, e->stream, e->codes_ring + slot * nq, (int)nq, e->sk_err,
-                       e->lx ? e->lx_err : nullptr, e->pin_out_dev);
-    SK_HIP(hipGetLastError());
+  if ((rc = enqueue_step(e, forced_codes != nullptr, logits_dbg)) != SK_OK) {
+    hipStreamSynchronize(e->stream);   // a launch that was queued may still read or write the pinned buffers
+    return rc;
   }
-  if (logits_dbg)
-    SK_HIP(hipMemcpyAsync(logits_dbg, e->dbg, nq * c.audio_vocab * sizeof(float), hipMemcpyDeviceToHost, e->stream));
   SK_HIP(hipStreamSynchronize(e->stream));
   memcpy(codes_out, e->pin_out, nq * sizeof(int64_t));
   e->fc_host += 1;

@@ -1,0 +1,64 @@
+"""The engine's host side on a stand-in HIP runtime (hip_host_stub.cpp), no GPU:
+what a failing call leaves behind, and which kernels a shape is given."""
+
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+HERE = os.path.join(ROOT, "tests")
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    d = tmp_path_factory.mktemp("hip")
+    so = str(d / "stub.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_host_stub.cpp"), "-o", so], check=True)
+
+    def run(script, **env):
+        f = d / "script.py"
+        f.write_text(script)
+        r = subprocess.run([sys.executable, os.path.join(HERE, "host_engine.py"), so, str(f)], capture_output=True,
+                           text=True, env=dict(os.environ, **env))
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+
+    return run
+
+
+STEP = """
+s = TINY
+h = engine(s)
+for r in range(2):
+    assert stage(h, s, r) == 0, error()
+assert L.sk_prefill_run(h) == 0 and L.sk_capture(h) == 0, error()
+codes = (C.c_int64 * s.n_codebooks)()
+logits = (C.c_float * (s.n_codebooks * s.audio_vocab))()
+step = lambda: L.sk_step_frame(h, 1, None, None, codes, logits)
+calls()
+"""
+
+
+@pytest.mark.parametrize("name,after", [("hipLaunchKernel", 0), ("hipGraphLaunch", 0), ("hipLaunchKernel", 1),
+                                        ("hipMemcpyAsync", 0)])
+def test_failing_step_waits_for_what_it_queued(host, name, after):
+    """A stepped frame that fails after its first launch waits for the stream
+    before it returns: that launch reads the pinned buffer which the next step
+    fills."""
+    host(STEP + f"""
+assert L.sk_set_debug(h, 1) == 0 and step() == 0, error()
+calls()
+stub.stub_fail(b"{name}", {after})
+rc = step()
+cs = [c[0] for c in calls()]
+assert rc == _lib.SK_EHIP, (rc, cs)
+text = error()
+assert "{name}" in cs and "stub error" in text, (cs, text)
+assert cs[-1] == "hipStreamSynchronize", cs
+stub.stub_fail(b"", -1)
+assert step() == 0, error()
+""")
