@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -1429,8 +1430,14 @@ int sk_prefill_row(sk_engine* e, int32_t row, const int64_t* text_ids, int32_t n
   SK_CHECK(c.n_language == 0 || n_text == 0 || e->lang, SK_ENOWEIGHT, "language_embeddings.weight is not bound");
   // Only kept here: the prefill embeds every staged row's tokens in one launch.
   const int n = n_text + n_frames;
-  e->ids_host[row].assign(text_ids, text_ids + n_text);
-  e->frames_host[row].assign(frame_codes, frame_codes + (size_t)n_frames * c.n_codebooks);
+  try {   // both copies before either takes the place of what the row has staged
+    std::vector<int> ids(text_ids, text_ids + n_text);
+    std::vector<int> codes(frame_codes, frame_codes + (size_t)n_frames * c.n_codebooks);
+    e->ids_host[row].swap(ids);
+    e->frames_host[row].swap(codes);
+  } catch (const std::bad_alloc&) {
+    return fail(SK_EHIP, "host memory for a prefix of %d tokens", n);
+  }
   e->len_host[row] = n;
   e->staged[row] = 1;
   e->prefilled = false;
@@ -1468,7 +1475,12 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
   size_t n_codes = 0;
   for (int r = 0; r < R; ++r)
     if (e->staged[r]) { M += e->len_host[r]; n_codes += e->frames_host[r].size(); }
-  std::vector<int> tab(2 * (size_t)R + 3 * (size_t)M + n_codes);
+  std::vector<int> tab;
+  try {
+    tab.resize(2 * (size_t)R + 3 * (size_t)M + n_codes);
+  } catch (const std::bad_alloc&) {
+    return fail(SK_EHIP, "host memory for a prefill of %d tokens", M);
+  }
   int* row_len = tab.data();
   int *row_start = row_len + R, *tok_row = row_start + R, *tok_pos = tok_row + M, *tok_src = tok_pos + M;
   int* codes = tok_src + M;

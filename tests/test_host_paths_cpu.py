@@ -62,3 +62,30 @@ assert cs[-1] == "hipStreamSynchronize", cs
 stub.stub_fail(b"", -1)
 assert step() == 0, error()
 """)
+
+
+def test_prefix_without_host_memory_is_refused(host):
+    """Prefixes are kept in host memory until the prefill runs: where there is
+    none, staging and the prefill report it (no C++ exception leaves the C
+    interface) and the engine goes on with what it had."""
+    host("""
+s = TINY
+h = engine(s)
+for r in range(2):
+    assert stage(h, s, r) == 0, error()
+stub.stub_new_limit(200)
+rc, text = stage(h, s, 1, 3, 30), error()
+assert rc == _lib.SK_EHIP and "host memory" in text, (rc, text)
+stub.stub_new_limit(-1)
+calls()
+assert L.sk_prefill_run(h) == 0, error()
+tokens = [g[0] for n, g in kernels(calls()) if "pf_embed" in n]
+assert tokens == [8], tokens            # two rows of 3 + 1 tokens, as staged before
+for r in range(2):
+    assert stage(h, s, r, 3, 30) == 0, error()
+stub.stub_new_limit(600)
+rc, text = L.sk_prefill_run(h), error()
+assert rc == _lib.SK_EHIP and "host memory" in text, (rc, text)
+stub.stub_new_limit(-1)
+assert L.sk_prefill_run(h) == 0, error()
+""")
