@@ -220,20 +220,27 @@ static hipError_t launch_depth_fused(const SampleArgs& s, const GemvArgs& g, int
 }
 
 // Depth steps by code tables (depth_step_kernel): one utterance's rows (2 with
-// CFG, 1 without) at the depth widths of the two trunk shapes.  Against the
-// launches per codebook they replace (SwiGLU with the sampler in front, down,
-// classifier), 0.6B BF16, one row: 14.6 -> 11.9 us.
+// CFG, 1 without) at the depth widths of the two trunk shapes, for every
+// vocabulary whose sampler fits in 64 KB of LDS (V <= 3,840 or so).  Against
+// the launches per codebook they replace (SwiGLU with the sampler in front,
+// down, classifier), 0.6B BF16, one row: 14.6 -> 11.9 us.
 static inline bool code_tables_fit(int d, int rows, int depth_inner, int V) {
-  return (rows == 1 || rows == 2) && (d == 1024 || d == 2048) && depth_inner == 2 * d && V <= 5 * SNT &&
+  return (rows == 1 || rows == 2) && (d == 1024 || d == 2048) && depth_inner == 2 * d && V <= MAX_V &&
          depth_sample_smem(V) <= 65536;
 }
 template <typename TL, int KD, int KI, int MODE, int M>
 static hipError_t launch_depth_step_t(const SampleArgs& s, const DepthArgs& g, int q, hipStream_t st) {
-  // 5 logits per thread cover the codebooks' V = 2,051 and anything smaller
-  constexpr int VPT = MODE == 2 ? 5 : 1;
-  hipLaunchKernelGGL((depth_step_kernel<TL, VPT, M, KD, KI, MODE>), dim3(DEPTH_WGS), dim3(SNT),
-                     MODE == 2 ? depth_sample_smem(s.V) : 0, st, s, g, q);
-  return hipGetLastError();
+  auto launch = [&](auto vpt, size_t smem) {
+    hipLaunchKernelGGL((depth_step_kernel<TL, decltype(vpt)::value, M, KD, KI, MODE>), dim3(DEPTH_WGS), dim3(SNT), smem,
+                       st, s, g, q);
+    return hipGetLastError();
+  };
+  // with a sampler: no more logits per thread than V needs (0.6B FP32 pair, us
+  // per frame with 5 for every V -> with its own: V = 512 751 -> 737, 1,024
+  // 759 -> 748, 1,536 760 -> 757; past 2,560, without tables -> with: 2,603
+  // 830 -> 782, 3,503 839 -> 786)
+  if constexpr (MODE == 2) return with_vpt(s.V, [&](auto vpt) { return launch(vpt, depth_sample_smem(s.V)); });
+  else return launch(std::integral_constant<int, 1>{}, 0);
 }
 template <typename TL, int MODE>
 static hipError_t launch_depth_step_w(int d, int rows, const SampleArgs& s, const DepthArgs& g, int q, hipStream_t st) {

@@ -89,3 +89,28 @@ assert rc == _lib.SK_EHIP and "host memory" in text, (rc, text)
 stub.stub_new_limit(-1)
 assert L.sk_prefill_run(h) == 0, error()
 """)
+
+
+@pytest.mark.parametrize("name,bf16", [("QWEN3_06B", False), ("QWEN3_06B", True), ("QWEN3_17B", False),
+                                       ("QWEN3_17B", True)])
+def test_code_table_vocabularies(host, name, bf16):
+    """Depth steps by code tables for every vocabulary whose sampler fits in
+    LDS, with no more logits per thread than it needs."""
+    out = host(f"""
+import re
+for rows in (1, 2):
+    for V in (100, 512, 513, 1024, 1025, 1536, 1537, 2051, 2560, 2561, 3840, 3841, 4096):
+        s = replace({name}, n_layers=1, n_codebooks=3, codebook_size=V - 3, text_vocab=64)
+        h = engine(s, cfg_rows=rows, bf16={bf16})
+        calls()
+        assert L.sk_capture(h) == 0, error()
+        steps = [re.search(r"depth_step_kernelI.*?Li(\\d+)ELi(\\d)ELi\\d+ELi\\d+ELi(\\d)E", n) for n, _ in kernels(calls())]
+        steps = [tuple(int(x) for x in m.groups()) for m in steps if m]
+        print(rows, V, sorted(set(p for p, m, mode in steps if mode == 2)), sorted(set(m for _, m, _ in steps)))
+        L.sk_destroy(h)
+""")
+    want = {100: 1, 512: 1, 513: 2, 1024: 2, 1025: 3, 1536: 3, 1537: 5, 2051: 5, 2560: 5, 2561: 8, 3840: 8}
+    for line in out.splitlines():
+        rows, V, rest = line.split(" ", 2)
+        n = want.get(int(V))
+        assert rest == (f"[{n}] [{rows}]" if n else "[] []"), line
