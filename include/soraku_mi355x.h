@@ -191,7 +191,7 @@ int32_t sk_frames_done(sk_engine* e);
 /* Diagnostic with no counterpart in the reference (which has one decode
  * path): 1 when the engine runs its trunk as XCD-resident layers (two
  * launches per layer; one or two decode rows at the Qwen3-0.6B or Qwen3-1.7B
- * trunk shape, on a device of 256 CUs, unless
+ * trunk shape but one FP32 row at the latter, on a device of 256 CUs, unless
  * SORAKU_XCD_LAYERS=0 was set at sk_create), 0 when it runs the per-op layer
  * kernels, -1 for a NULL engine.  For tests and profiling. */
 int32_t sk_xcd_layers(sk_engine* e);

@@ -481,9 +481,15 @@ hipError_t launch_attn_stream(sk_engine* e, const AttnArgs& at) {
 
 // XCD-resident layers (sk_layer.h): one or two decode rows, 16 q / 8 KV heads
 // of 128, at the Qwen3-0.6B trunk shape (d 1024, SwiGLU 3072) or the
-// Qwen3-1.7B one (d 2048, SwiGLU 6144), FP32 or BF16 weights and cache.
+// Qwen3-1.7B one (d 2048, SwiGLU 6144), FP32 or BF16 weights and cache; one
+// row at 1.7B with BF16 weights only.  us per frame of one row, five kernels
+// per layer / these, contexts of 58 and 700: 0.6B FP32 911 / 741 and 992 /
+// 823, BF16 800 / 646 and 887 / 725; 1.7B BF16 1,138 / 1,096 and 1,228 /
+// 1,173, FP32 1,601 / 2,473 and 1,690 / 2,554 (its MLP half's weights do not
+// fit in the registers: 220 bytes of scratch per lane).
 bool lx_fits(const sk_engine* e) {
   const sk_config& c = e->c;
+  if (e->rows == 1 && c.d_model == 2048 && c.weight_dtype != SK_BF16) return false;
   const bool shape = (c.d_model == 1024 && c.trunk_inter == 3072) || (c.d_model == 2048 && c.trunk_inter == 6144);
   // n_layers % 3 == 2 would leave the trunk's output in accumulator 1, the
   // next frame's first-layer target, which the frame's last launch must zero

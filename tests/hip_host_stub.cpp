@@ -65,7 +65,11 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStr
 hipError_t hipGetLastError() { const hipError_t e = last_launch; last_launch = hipSuccess; return e; }
 const char* hipGetErrorString(hipError_t) { return "stub error"; }
 
-hipError_t hipMalloc(void** p, size_t n) { *p = aligned_alloc(256, (n + 255) & ~(size_t)255); return note("hipMalloc", " " + std::to_string(n)); }
+hipError_t hipMalloc(void** p, size_t n) {
+  *p = aligned_alloc(256, (n + 255) & ~(size_t)255);
+  if (*p && n < (1u << 20)) memset(*p, 0, n);   // small ones may be read back (the XCD probe's ids)
+  return note("hipMalloc", " " + std::to_string(n));
+}
 hipError_t hipFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(1, n); return note("hipHostMalloc"); }
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }

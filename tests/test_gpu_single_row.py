@@ -1,5 +1,5 @@
-"""Decode rows and widths that the XCD-resident layers and the code-table depth
-steps take beside the CFG pair in FP32 (0.6B) and BF16 (1.7B): one row without
+"""Decode rows and widths that the XCD-resident layers (all but one FP32 row at
+d 2048) and the code-table depth steps take beside the CFG pair in FP32 (0.6B) and BF16 (1.7B): one row without
 CFG (beside an inactive row of zeros), BF16 weights at d 1024 (half-width inner
 pieces), FP32 weights at d 2048 (double-width ones).  Four trunk layers of the
 real widths, teacher-forced frames against the float64 oracle; a second prefill
@@ -57,7 +57,7 @@ def test_row_counts_and_widths_match_oracle(hip_device, name, rows, bf16):
     codes, u = rng.integers(0, V, (F, Q)), rng.random((F, Q))
     print(f"{name} rows {rows} bf16 {bf16}", flush=True)
     e = _engine(hip_device, s, w, rows, bf16)
-    assert e.xcd_layers
+    assert e.xcd_layers == (not (name == "17b" and rows == 1 and not bf16))   # that one keeps five kernels per layer
     got = _frames(e, items[0], codes, u)
     m = om.OracleModel(s, w, np.float64)
     rec = Record()

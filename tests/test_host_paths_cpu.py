@@ -114,3 +114,21 @@ for rows in (1, 2):
         rows, V, rest = line.split(" ", 2)
         n = want.get(int(V))
         assert rest == (f"[{n}] [{rows}]" if n else "[] []"), line
+
+
+def test_xcd_layers_rule(host):
+    """Which engines run the XCD-resident layers."""
+    out = host("""
+for name, s in (("06b", QWEN3_06B), ("17b", QWEN3_17B)):
+    for rows in (1, 2, 3):
+        for bf16 in (False, True):
+            h = engine(replace(s, n_layers=3, n_codebooks=2, text_vocab=64), n_utts=3 if rows == 3 else 1,
+                       cfg_rows=1 if rows == 3 else rows, bf16=bf16)
+            print(name, rows, bf16, L.sk_xcd_layers(h))
+            L.sk_destroy(h)
+""")
+    got = {tuple(line.split()[:3]): line.split()[3] for line in out.splitlines()}
+    assert len(got) == 12
+    for (name, rows, bf16), lx in got.items():
+        want = rows == "2" or (rows == "1" and (name == "06b" or bf16 == "True"))
+        assert lx == str(int(want)), (name, rows, bf16, lx)
