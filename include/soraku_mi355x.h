@@ -193,7 +193,9 @@ int32_t sk_frames_done(sk_engine* e);
  * launches per layer; one or two decode rows at the Qwen3-0.6B or Qwen3-1.7B
  * trunk shape but one FP32 row at the latter, on a device of 256 CUs, unless
  * SORAKU_XCD_LAYERS=0 was set at sk_create), 0 when it runs the per-op layer
- * kernels, -1 for a NULL engine.  For tests and profiling. */
+ * kernels, -1 for a NULL engine.  These layers hold the residual stream in
+ * units of 2^-32 (64 bits): a residual row with a norm of 2^27 or more becomes
+ * NaN, as one that holds NaN or infinity does. */
 int32_t sk_xcd_layers(sk_engine* e);
 /* Test hook with no counterpart in the reference: the bound, in ticks of the
  * 100 MHz real-time counter, of every wait inside a frame's kernels (the

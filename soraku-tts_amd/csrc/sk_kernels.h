@@ -2511,6 +2511,12 @@ __device__ __forceinline__ float2 rope_cs(int p, float fq) {
   return make_float2((float)cos((double)ang), (float)sin((double)ang));
 }
 
+// The sum of squares of a row (or half of one) of the fixed-point residual
+// stream (2^-32 units in 64 bits): NaN from 2^54 on, where a value may be out of
+// the stream's range (sk_layer.h, lx_accum).
+constexpr float FIX_SS_MAX = 0x1p54f;
+__device__ __forceinline__ float fix_range(float ss) { return ss < FIX_SS_MAX ? ss : __uint_as_float(0x7fc00000u); }
+
 // ------------------------------------------------------------ depth step (code tables)
 // One utterance's depth step (M = 2 rows with CFG, 1 without) with the SwiGLU
 // input taken apart by linearity.
@@ -2812,7 +2818,7 @@ __global__ __launch_bounds__(SNT) void depth_step_kernel(SampleArgs a, DepthArgs
       float t = 0.f;
 #pragma unroll
       for (int w = 0; w < SWAVES; ++w) t += red[m][w];
-      const float invf = 1.0f / sqrtf(t / (float)KD + g.fnorm_eps);
+      const float invf = 1.0f / sqrtf((TFIX ? fix_range(t) : t) / (float)KD + g.fnorm_eps);
 #pragma unroll
       for (int i = 0; i < DPT; ++i) {
         const float h = fw[i] * (hv[m][i] * invf);
@@ -3091,6 +3097,9 @@ __global__ __launch_bounds__(NT) void final_norm_kernel(const float* x, const lo
     u0 = u_ring[(size_t)nx * nq + min(tx, nq - 1)];
     f0 = flag_ring[2 * nx + min(tx, 1)];
   };
+  auto inv_rms = [&](float ss) {
+    return 1.0f / sqrtf((xfix ? fix_range(ss) : ss) / (float)D + eps);
+  };
   if (!act) book();
   if (!act && fix_clear)   // a retired row's entries too: a refill may make it active again
     for (int i = tx; i < D; i += NT) fix_clear[(size_t)b * D + i] = 0ull;
@@ -3136,7 +3145,7 @@ __global__ __launch_bounds__(NT) void final_norm_kernel(const float* x, const lo
 #pragma unroll
       for (int i = 0; i < P4; ++i)
         if (i < n4) s += xv[i].x * xv[i].x + xv[i].y * xv[i].y + xv[i].z * xv[i].z + xv[i].w * xv[i].w;
-      const float inv = 1.0f / sqrtf(block_sum(s, red) / (float)D + eps);
+      const float inv = inv_rms(block_sum(s, red));
       if (fix_clear) {   // every thread's loads are consumed: the row may be the one read
         ulonglong2* c2 = reinterpret_cast<ulonglong2*>(fix_clear + ro);
 #pragma unroll
@@ -3189,7 +3198,7 @@ __global__ __launch_bounds__(NT) void final_norm_kernel(const float* x, const lo
 #pragma unroll
       for (int i = 0; i < PER; ++i)
         if ((int)threadIdx.x + i * NT < D) s += xv[i] * xv[i];
-      const float inv = 1.0f / sqrtf(block_sum(s, red) / (float)D + eps);
+      const float inv = inv_rms(block_sum(s, red));
       if (fix_clear) {
 #pragma unroll
         for (int i = 0; i < PER; ++i)
@@ -3222,7 +3231,7 @@ __global__ __launch_bounds__(NT) void final_norm_kernel(const float* x, const lo
       book();
       float s = 0.f;
       for (int k = threadIdx.x; k < D; k += NT) s += xr[k] * xr[k];
-      const float inv = 1.0f / sqrtf(block_sum(s, red) / (float)D + eps);
+      const float inv = inv_rms(block_sum(s, red));
       float s2 = 0.f;
       for (int k = threadIdx.x; k < D; k += NT) {
         const float h = w[k] * (xr[k] * inv);

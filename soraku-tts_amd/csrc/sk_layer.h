@@ -226,13 +226,25 @@ __device__ __forceinline__ bool lx_xcd_barrier(unsigned* fl, int j, unsigned tar
 
 // Fixed-point residual stream: value * 2^32 in a 64-bit integer.  FP32 to
 // fixed point drops only bits below 2^-32; fixed point to FP32 rounds once.
+//
+// What has no fixed-point value (NaN, infinity, a partial of 2^24 or more)
+// makes the row NaN from there on, as it does in FP32 arithmetic: such a
+// partial adds LX_BAD = 2^64 / 10 and drops x.  An output's 8 partials and x
+// (in range below 2^59 units, see FIX_SS_MAX; a partial below 2^56) then sum,
+// modulo 2^64, to a multiple 1 .. 8 of LX_BAD and less than 2^60 beside it,
+// always at least 2^59 units from zero, so the next reader sees a sum of
+// squares out of range, takes it as NaN, and every partial after that is NaN.
+// (Checked on the sum of squares, the input costs one compare per wave.)
 constexpr float LX_FIX_ONE = 4294967296.0f;
+constexpr float LX_PART_MAX = 16777216.0f;
+constexpr long long LX_BAD = 1844674407370955161ll;
 __device__ __forceinline__ long long lx_fix(float v) { return (long long)(v * LX_FIX_ONE); }
 __device__ __forceinline__ float lx_unfix(long long q) { return (float)q * (1.0f / LX_FIX_ONE); }
 // Partial v of output (m, n), plus x (fixed point) on XCD 0, into the next
 // accumulator.
 __device__ __forceinline__ void lx_accum(unsigned long long* acc, size_t idx, float v, long long x) {
-  __hip_atomic_fetch_add(acc + idx, (unsigned long long)(lx_fix(v) + x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const long long q = fabsf(v) < LX_PART_MAX ? lx_fix(v) + x : LX_BAD;
+  __hip_atomic_fetch_add(acc + idx, (unsigned long long)q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Input of a launch, loaded by the stream waves (threads 256..511): stream
@@ -297,7 +309,7 @@ struct LxIn {
 #pragma unroll
       for (int k = 0; k < 4; ++k) ss = fmaf(v[4 * i + k], v[4 * i + k], ss);
     }
-    ss = wave_sum_dpp(ss);
+    ss = fix_range(wave_sum_dpp(ss));
     if ((st & 63) == 0) ssq[w4] = ss;
   }
 };
