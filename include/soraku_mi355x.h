@@ -195,7 +195,7 @@ int32_t sk_frames_done(sk_engine* e);
  * SORAKU_XCD_LAYERS=0 was set at sk_create), 0 when it runs the per-op layer
  * kernels, -1 for a NULL engine.  These layers hold the residual stream in
  * units of 2^-32 (64 bits): a residual row with a norm of 2^27 or more becomes
- * NaN, as one that holds NaN or infinity does. */
+ * NaN, as one that holds NaN or infinity does.  For tests and profiling. */
 int32_t sk_xcd_layers(sk_engine* e);
 /* Test hook with no counterpart in the reference: the bound, in ticks of the
  * 100 MHz real-time counter, of every wait inside a frame's kernels (the

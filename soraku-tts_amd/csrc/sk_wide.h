@@ -313,7 +313,13 @@ __global__ __launch_bounds__(W * 64) void skinny_kernel(SkinnyArgs a) {
   const int kw0 = kbeg + wave * BK;
   const int nst = kw0 < kend ? (kend - kw0 + STEP - 1) / STEP : 0;
   constexpr int SREG = XS ? 4 * NA + 8 * TR : (NA + (TR + (XNORM ? 1 : 0)) * NX) * 4;   // registers of a stage
-  constexpr int UP = SREG > 20 || (MM <= MM_XS && TR == 2) ? 4 : 8, CH = UP / 2;
+  // Registers of 8 stages, the sums and the operands in work: past 224 of the
+  // 256 that a lane of 8 waves has, the compiler spills.  4 stages instead of 8
+  // with spills: FP32 gate/up, 18 / 20 / 32 rows, 0.6B frame 1,852 / 1,901 /
+  // 2,091 us -> 1,832 / 1,882 / 2,071 (6 stages 1,885 / 1,935 / 2,107); BF16
+  // operators of 20 rows, 1024 x 3080 14.8 -> 12.2 us, 2048 x 6136 25.0 -> 20.8.
+  constexpr int REGS8 = 8 * SREG + (EXACT ? (NACC + 1) * NA * TR * 4 + TR * VEC + (TAIL ? 2 * VEC : 0) : 0);
+  constexpr int UP = SREG > 20 || (MM <= MM_XS && TR == 2) ? 4 : REGS8 > 224 ? 4 : 8, CH = UP / 2;
   auto upfront = [&](int k0, auto nc) __attribute__((always_inline)) {
     constexpr int NC = decltype(nc)::value;
     Stage st[NC];
