@@ -128,7 +128,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs a) {
   const bool odd = a.K % KS != 0;
   const int s0 = st_all * ks / a.ksplit, nst = st_all * (ks + 1) / a.ksplit - s0;
 
-  // loader: group g of the stage = 16 rows x 128 bytes, two 1 KB pieces;
+  // loader: group g of the stage = 16 rows x H pieces of 64 bytes (1 KB each);
   // scalar base per group (its first row), the lane's row and 16 bytes in voff
   const char* gb[CPW];
   unsigned voff[CPW];
@@ -314,7 +314,7 @@ inline GemmPlan plan_gemm(bool bf16, bool swiglu, int M, int N, int K, int max_s
     const int nc = swiglu ? g.bn / 2 : g.bn;
     const long tiles = (long)((M + g.bm - 1) / g.bm) * ((N + nc - 1) / nc);
     for (int ks : {1, 2, 3, 4, 6, 8, 12, 16}) {
-      if (ks > max_split || units < 4 * ks) break;
+      if (ks > 1 && (ks > max_split || units < 4 * ks)) break;   // (short K: one slice, of the tile that fits M and N)
       const long rounds = (tiles * ks + 255) / 256;
       const float us = g.fix + rounds * g.round + ((units + ks - 1) / ks) * (g.lat + (rounds - 1) * g.thr) +
                        (ks - 1) * ((float)M * N * 8e-6f / 6.f + .1f);

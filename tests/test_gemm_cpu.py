@@ -45,3 +45,30 @@ __global__ void k(const char* g, float* out, int v) {
     after = body[body.index("global_load_lds_dwordx4"):]
     after = after[:re.search(r"s_sendmsg|global_load_lds_dword ", after).start()]
     assert re.search(r"s_\w+ m0,", after), body
+
+
+def test_plan_evaluates_every_tile_for_short_k(tmp_path):
+    """K of fewer than four 64-byte units still gets the tile with the smallest
+    estimate, in one slice (not whichever comes first in the table)."""
+    exe = _hipcc(tmp_path, """
+#include <stdio.h>
+#include "sk_gemm.h"
+int main() {
+  for (int bf = 0; bf < 2; ++bf)
+    for (int sw = 0; sw < 2; ++sw)
+      for (int K : {32, 64, 96, 128})
+        for (int M : {2, 40, 300, 5000}) {
+          const sk::GemmPlan p = sk::plan_gemm(bf, sw, M, 160, K, 16);
+          const sk::GemmTile t = bf ? sk::GEMM_BF16[p.tile] : sk::GEMM_F32[p.tile];
+          printf("%d %d %d %d %d %d %d %d\\n", bf, sw, K, M, t.bm, t.bn, (int)t.swiglu, p.ksplit);
+        }
+}
+""", "--offload-host-only")
+    out = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
+    rows = [tuple(int(x) for x in line.split()) for line in out.splitlines()]
+    assert len(rows) == 64
+    for bf, sw, K, M, bm, bn, ok, ks in rows:
+        assert ks == 1 or K * (2 if bf else 4) >= 4 * 64 * ks, (bf, sw, K, M, ks)
+        assert ok or not sw
+        if M <= 40:
+            assert bm <= 64 and bn <= 128, (bf, sw, K, M, bm, bn)   # not a tile 4 times the rows
