@@ -1,8 +1,8 @@
-"""The batched prefill over the range of its GEMM tiles and K slices: prefixes
-of a few to a thousand tokens in several ragged rows against the float64
-oracle.  The token counts sit at and around the tile heights (32 .. 256 rows),
-the widths take the trunk shapes and an odd one whose K ends in half a stage
-(K = 96: 64-byte units of BF16 and FP32 rows).
+"""The batched prefill over K slices and the smaller GEMM tiles: prefixes of a
+few to a thousand tokens in several ragged rows against the float64 oracle.  The
+token counts sit at and around the tile heights, the widths take the trunk
+shapes and an odd one with short K (96 and 160); test_gpu_prefill_tiles.py has a
+case for every tile.
 
 Bounds: FP32 sums of K = 6144 products in another order differ by ~sqrt(K) *
 2^-24 = 5e-6 of a row's size per projection, 2e-5 over two layers; with BF16

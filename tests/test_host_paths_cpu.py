@@ -132,3 +132,37 @@ for name, s in (("06b", QWEN3_06B), ("17b", QWEN3_17B)):
     for (name, rows, bf16), lx in got.items():
         want = rows == "2" or (rows == "1" and (name == "06b" or bf16 == "True"))
         assert lx == str(int(want)), (name, rows, bf16, lx)
+
+
+def test_prefill_gemms_have_gpu_cases(host):
+    """Every GEMM kernel (epilogue, weight type, tile) that a prefill launches
+    at either trunk shape, up to 6,000 tokens, is launched by a case of
+    test_gpu_prefill_tiles.py; the short shape's cases reach the half stage."""
+    host("""
+import re
+import test_gpu_prefill_tiles as t
+
+def gemms(shape, lens, bf16):
+    h = engine(shape, n_utts=len(lens), cfg_rows=1, max_ctx=max(lens) + 4, bf16=bf16)
+    for r, n in enumerate(lens):
+        assert stage(h, shape, r, n - 1, 1) == 0, error()
+    calls()
+    assert L.sk_prefill_run(h) == 0, error()
+    names = [re.search(r"gemm_kernelILi(\\d)E.*?(WF32|WBF16)E((?:Li\\d+E)+)", n) for n, _ in kernels(calls())]
+    L.sk_destroy(h)
+    return {m.groups() for m in names if m}
+
+fields = [f.name for f in dataclasses.fields(QWEN3_06B)]
+tested = {}
+for name, total, bf16 in t.CASES:
+    s = replace(QWEN3_06B, **{f: getattr(t.shape(name), f) for f in fields})
+    tested.setdefault(name, set()).update(gemms(s, t.lens_of(total), bf16))
+used = set()
+for s in (QWEN3_06B, QWEN3_17B):
+    for total in list(range(16, 400, 9)) + list(range(400, 6000, 75)):
+        for bf16 in (False, True):
+            used |= gemms(replace(s, n_layers=1, text_vocab=512), t.lens_of(total), bf16)
+assert len(used) >= 28 and used <= tested["ragged"], used - tested["ragged"]
+half = {k for k in tested["short"] if k[2].endswith("Li2E")}
+assert {k[0] for k in half} == {"0", "1"}, half      # stages of 128 bytes, both epilogues
+""")
