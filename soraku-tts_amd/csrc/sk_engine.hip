@@ -1167,10 +1167,22 @@ int sk_create(const sk_config* cfg, void* hip_stream, sk_engine** out) {
   //   8 rows BF16 (cache too), 400 1: 1389, 4: 1408; 800 1: 1515, 4: 1437
   //   12 rows BF16, 240 1: 1350, 2: 1430, 3: 1592; 960 1: 1591, 2: 1547, 3: 1721
   //   20 rows FP32, 400 1: 2057, 2: 2294; 1600 1: 2879, 2: 2963
+  // 17 to 31 rows, where one split fits and two do not: two all the same for
+  // capacities from which on the second round's better balance (rows of half to
+  // all of the length) wins, the later the emptier that round is.  BF16 weights,
+  // 1 split / 2, by the cache's type and length:
+  //   17 rows BF16 16000 7264 / 7246, 50000 19815 / 19048; FP32 16000 11014 / 11332
+  //   21 rows BF16 40000 16368 / 16315; FP32 6000 5440 / 5649, 16000 12169 / 12452
+  //   24 rows BF16 6000 3926 / 3936, 16000 7961 / 7925, 50000 21845 / 20895; FP32 1600 2588 / 2742, 6000 5981 / 5761
+  //   28 rows BF16 6000 4233 / 4096; FP32 3000 3981 / 3822, 6000 6561 / 6343
+  //   31 rows BF16 6000 4316 / 4342, 16000 9214 / 9006; FP32 3000 4233 / 4155, 6000 7249 / 6804
   if (e->wide && (e->G == 1 || e->G == 2 || e->G == 4) && e->G * c.head_dim <= ATTN_STREAM_NTH) {
     const int pairs = e->rows * c.n_kv_heads;
     const size_t head_bytes = 2 * (size_t)c.max_ctx * c.head_dim * (c.kv_dtype == SK_BF16 ? 2 : 4);
-    e->attn_splits = head_bytes <= 256 * 1024 ? 1 : std::max(1, std::min(e->max_chunks, 256 / pairs));
+    const size_t two_mb = pairs < 176 ? 18 : pairs < 208 ? 6 : 3;
+    int splits = head_bytes <= 256 * 1024 ? 1 : 256 / pairs;
+    if (pairs > 128 && pairs < 256 && head_bytes > two_mb << 20) splits = 2;
+    e->attn_splits = std::max(1, std::min(e->max_chunks, splits));
   }
   e->L.resize(c.n_layers);
   e->kv_host.assign(e->rows, 0);

@@ -33,12 +33,12 @@ def _inputs(utts):
     return items, rng.integers(0, V, (F, utts, Q)), rng.random((F, utts, Q))
 
 
-def _run(dev, w, utts, max_len, items, codes, u, bf16=False):
+def _run(dev, w, utts, max_len, items, codes, u, bf16=False, shape=S):
     from soraku_amd import GraphFrameEngine
     from soraku_amd.config import DecodeShape
 
     e = GraphFrameEngine(device=dev, max_cache_len=max_len, cfg_scale=1.5, batch=2, state_dict=w,
-                         shape=DecodeShape(**{k: getattr(S, k) for k in DecodeShape.__dataclass_fields__}),
+                         shape=DecodeShape(**{k: getattr(shape, k) for k in DecodeShape.__dataclass_fields__}),
                          n_utts=utts, bf16=bf16, kv_bf16=bf16, max_frames=8)
     e.set_temperature(0.9)
     e.set_sampling(sampled=True, top_k=50, top_p=0.95)
@@ -79,3 +79,28 @@ def test_split_rule_bf16_cache(hip_device):
     fin = np.isfinite(one)
     assert (np.isfinite(split) == fin).all()
     assert np.abs(one[fin] - split[fin]).max() < 1e-3 * np.abs(one[fin]).max()
+
+
+@pytest.mark.parametrize("utts,max_len", [(9, 18500), (11, 6100), (11, 6200), (14, 3000), (14, 3100)])
+def test_two_splits_for_long_caches_match_oracle(hip_device, utts, max_len):
+    """18, 22 and 28 rows on both sides of the capacity from which two
+    workgroups share a row (18 rows: past it)."""
+    s = om.Shape(n_layers=1, text_vocab=512, n_codebooks=4)
+    w = om.synthetic_weights(s, 23, norm_gain_std=0.1, bias_std=0.02)
+    rng = np.random.default_rng(7)
+    items = [(rng.integers(0, 512, 20 + 9 * i), np.array([1], np.int64), rng.integers(0, s.codebook_size, (190 - 13 * i, 4)))
+             for i in range(utts)]
+    codes, u = rng.integers(0, s.codebook_size, (F, utts, 4)), rng.random((F, utts, 4))
+    print(f"utts {utts} capacity {max_len}", flush=True)
+    got = _run(hip_device, w, utts, max_len, items, codes, u, shape=s)
+    m = om.OracleModel(s, w, np.float64)
+    for i in (0, utts - 1):
+        rec = Record()
+        generate(m, input_ids=items[i][0], prompt_codes=items[i][2], uncond_input_ids=items[i][1], max_new_frames=F,
+                 min_new_frames=F, temperature=0.0, cfg_scale=1.5, batched=True, record=rec, forced_codes=codes[:, i])
+        for f in range(F):
+            ref = np.stack([apply_masks(x, q=q, frame_index=f, min_new_frames=F, bos_id=s.bos_id, eos_id=s.eos_id,
+                                        pad_id=s.pad_id) for q, x in enumerate(rec.merged[f])]).astype(np.float64)
+            fin = np.isfinite(ref)
+            assert (np.isfinite(got[f, i]) == fin).all()
+            assert np.abs(got[f, i][fin] - ref[fin]).max() < 2e-5 * np.abs(ref[fin]).max()

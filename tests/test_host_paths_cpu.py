@@ -166,3 +166,24 @@ assert len(used) >= 28 and used <= tested["ragged"], used - tested["ragged"]
 half = {k for k in tested["short"] if k[2].endswith("Li2E")}
 assert {k[0] for k in half} == {"0", "1"}, half      # stages of 128 bytes, both epilogues
 """)
+
+
+def test_attention_split_rule(host):
+    """Workgroups per (row, KV head) of the many-row attention: one for short
+    caches, else as many as fit 256 CUs; 17 to 31 rows two for long caches."""
+    out = host("""
+for rows, ctx, kv_bf16 in ((6, 256, 0), (6, 257, 0), (8, 640, 0), (8, 513, 1), (12, 640, 0), (16, 640, 0), (32, 65536, 1),
+                           (17, 2000, 0), (17, 18432, 0), (17, 18433, 0), (21, 36864, 1), (21, 36865, 1),
+                           (22, 6144, 0), (22, 6145, 0), (25, 12288, 1), (25, 12289, 1),
+                           (26, 3072, 0), (26, 3073, 0), (31, 6144, 1), (31, 6145, 1)):
+    s = replace(QWEN3_06B, n_layers=1, n_codebooks=2, text_vocab=64)
+    h = engine(s, n_utts=rows, cfg_rows=1, max_ctx=ctx, kv_bf16=bool(kv_bf16))
+    calls()
+    assert L.sk_capture(h) == 0, error()
+    grids = [g for n, g in kernels(calls()) if "attention_stream_kernel" in n]
+    assert len(grids) == 1 and grids[0][1:] == (8, rows), grids
+    print(rows, ctx, kv_bf16, grids[0][0])
+    L.sk_destroy(h)
+""")
+    got = [int(line.split()[3]) for line in out.splitlines()]
+    assert got == [1, 5, 4, 4, 2, 2, 1, 1, 1, 2, 1, 2, 1, 2, 1, 2, 1, 2, 1, 2], out
