@@ -105,3 +105,28 @@ def test_fp32_many_rows_match_oracle(hip_device, utts):
             fin = np.isfinite(ref[f])
             assert (np.isfinite(got[f][u]) == fin).all()
             assert np.abs(got[f][u][fin] - ref[f][fin]).max() / np.abs(ref[f][fin]).max() < 5e-5
+
+
+@pytest.mark.parametrize("B", [5, 16, 17, 32])
+@pytest.mark.parametrize("K,N", [(1024, 2051), (3080, 48), (6144, 96)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_rows_ops_keep_fp32_products(hip_device, B, K, N, bf16):
+    """The products are exact: errors stay at those of FP32 sums of at most 32
+    products in a row, a few 2^-24 of an output's RMS.  A hi + lo split of the
+    activations (2.4e-6) does not pass, nor, at the larger K, one sum per wave
+    (3.7e-7 and more)."""
+    import torch
+
+    from soraku_amd import ops
+
+    rng = np.random.default_rng(B + K)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    x = rng.standard_normal((B, K), dtype=np.float32)
+    w = rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05)
+    w = om.round_bf16(w) if bf16 else w
+    ref = x.astype(np.float64) @ w.T.astype(np.float64)
+    zero = torch.zeros(N, device=hip_device)
+    got = ops.classifier_gemv(B, N, K)(torch.from_numpy(x).to(hip_device), torch.from_numpy(w).to(hip_device, dt), zero)
+    err = np.sqrt(np.mean((got.cpu().numpy() - ref) ** 2) / np.mean(ref ** 2))
+    print(f"B={B} K={K} N={N} bf16={bf16}: {err:.2e}", flush=True)
+    assert err < 2e-7   # 24 totals of 32 products: 2^-24 * 0.4 * (sqrt(32 / 2) + sqrt(24 / 2)) = 1.8e-7; measured 1.0e-7 to 1.35e-7
