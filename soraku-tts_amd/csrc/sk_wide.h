@@ -580,14 +580,25 @@ inline hipError_t launch_skinny_w(bool bf16, const SkinnyArgs& a, bool allow_spl
 }
 
 // The operator API's projections of at most 32 rows: exact products, any N, K
-// a multiple of 8.  SwiGLU of up to 16 rows in workgroups of 4 waves (three per
-// CU, so one loads while another multiplies: 7 rows, BF16 2 x 6144 x 2048, 18.3 us
-// against 30.4 us with 8 waves), the rest, with half the tiles, of 8 (2048 x
-// 6144: 15.2 us against 19.6 with 4 and 22.5 with 16).
+// a multiple of 8, in workgroups of 8 waves.  SwiGLU of up to 16 rows takes 4
+// waves where that was faster: more than 256 output tiles, so that a CU holds
+// two workgroups (232 registers; one where K has a tail) and one loads while the
+// other multiplies, and wide FP32 rows.  us of a launch, 7 rows, gate and up,
+// 4 waves / 8: BF16 2048 x 1024 7.0 / 5.7, 2688 x 1344 8.9 / 7.0, 4096 x 2048
+// 12.0 / 11.2, 4608 x 1536 13.9 / 14.8, 6144 x 2048 16.4 / 20.7; FP32 2000 x 1000
+// 7.2 / 6.5, 3072 x 1024 7.4 / 7.1, 2688 x 1344 9.3 / 9.5, 4096 x 2048 13.7 /
+// 14.3, 6144 x 2048 22.2 / 24.1; 5, 11 and 16 rows the same way round.  (The
+// others, BF16 2048 x 6144: 8 waves 15.2, 4 waves 19.6, 16 waves 22.5.)
 template <int EPI, int MM, int TR, bool TAIL>
 inline hipError_t launch_rows_t(const SkinnyArgs& a, hipStream_t st) {
-  constexpr int W = EPI == EPI_SWIGLU && TR == 1 ? 4 : 8;
-  hipLaunchKernelGGL((skinny_kernel<EPI, W, false, MM, TR, TAIL>), dim3((a.N + 15) / 16), dim3(W * 64), 0, st, a);
+  const int tiles = (a.N + 15) / 16;
+  if constexpr (EPI == EPI_SWIGLU && TR == 1) {
+    if (tiles > 256 || (MM == MM_F32 && a.K > 1024)) {
+      hipLaunchKernelGGL((skinny_kernel<EPI, 4, false, MM, TR, TAIL>), dim3(tiles), dim3(4 * 64), 0, st, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((skinny_kernel<EPI, 8, false, MM, TR, TAIL>), dim3(tiles), dim3(8 * 64), 0, st, a);
   return hipGetLastError();
 }
 template <int EPI, int MM>

@@ -130,3 +130,26 @@ def test_rows_ops_keep_fp32_products(hip_device, B, K, N, bf16):
     err = np.sqrt(np.mean((got.cpu().numpy() - ref) ** 2) / np.mean(ref ** 2))
     print(f"B={B} K={K} N={N} bf16={bf16}: {err:.2e}", flush=True)
     assert err < 2e-7   # 24 totals of 32 products: 2^-24 * 0.4 * (sqrt(32 / 2) + sqrt(24 / 2)) = 1.8e-7; measured 1.0e-7 to 1.35e-7
+
+
+@pytest.mark.parametrize("B", [5, 16, 17])
+@pytest.mark.parametrize("K,N", [(256, 4096), (256, 4097), (264, 4100), (1024, 96), (1032, 96), (1040, 96)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_swiglu_workgroup_rule_matches_float64(hip_device, B, K, N, bf16):
+    """SwiGLU on both sides of the rule for 4 or 8 waves: 256 output tiles, K of
+    1,024 with FP32 weights, whole blocks and tails.  Bound: of the operators
+    above, products of two sums each good to ~3e-6 of the largest."""
+    import torch
+
+    from soraku_amd import ops
+
+    rng = np.random.default_rng(B * 31 + K + N)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    x = rng.standard_normal((B, K), dtype=np.float32)
+    ws = [rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05) for _ in range(2)]
+    ws = [om.round_bf16(w) if bf16 else w for w in ws]
+    print(f"swiglu B={B} K={K} N={N} bf16={bf16}", flush=True)
+    got = ops.swiglu_gemv(B, N, K)(torch.from_numpy(x).to(hip_device),
+                                   *(torch.from_numpy(w).to(hip_device, dt) for w in ws)).cpu().numpy()
+    g, u = (x.astype(np.float64) @ w.T.astype(np.float64) for w in ws)
+    assert _rel(got, om.silu(g) * u) < 2e-5
