@@ -87,14 +87,15 @@ size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Bytes of PrefillBufs for M tokens, each buffer 256-byte aligned, and where
 // QKV's share goes: one slice, or for few tokens (whose GEMMs need their K cut
 // to fill the GPU) up to 4 MB of slices, as long as that alone does not push
-// the prefill past the scratch of sk_prefill_run_noalloc.
+// the prefill past the scratch of sk_prefill_run_noalloc.  QKV also has 8 bytes
+// per token beyond its slices, which keep the largest prefill that fits there
+// what it is.
 struct PrefillSizes { size_t qkv, total; };
 PrefillSizes prefill_sizes(const sk_config& c, int nqkv, size_t M) {
-  const size_t hq = (size_t)c.n_q_heads * c.head_dim;
-  const size_t rest = up256(M * c.d_model * 4) * 2 + up256(M * hq * 4) * 2 + up256(M * c.trunk_inter * 4) +
-                      up256(M * 4) * 2;   // (two token tables, now elsewhere: the size that fits stays what it was)
-  const size_t one = up256(M * nqkv * 4), room = SK_NOALLOC_SCRATCH_BYTES;
-  size_t qkv = std::max(one, std::min<size_t>(4u << 20, rest < room ? (room - rest) & ~(size_t)255 : 0));
+  const size_t hq = (size_t)c.n_q_heads * c.head_dim, room = SK_NOALLOC_SCRATCH_BYTES;
+  const size_t rest = up256(M * c.d_model * 4) * 2 + up256(M * hq * 4) * 2 + up256(M * c.trunk_inter * 4);
+  const size_t extra = up256(M * 4) * 2, one = up256(M * nqkv * 4), used = rest + extra;
+  const size_t qkv = extra + std::max(one, std::min<size_t>(4u << 20, used < room ? (room - used) & ~(size_t)255 : 0));
   return PrefillSizes{qkv, rest + qkv};
 }
 

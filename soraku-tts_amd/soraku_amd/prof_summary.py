@@ -46,7 +46,7 @@ def short_name(name: str) -> str:
     return n.strip()
 
 
-PREFILL_MARKERS = ("prefill", "pf_", "gemm_nt_kernel", "gemm_kernel")
+PREFILL_MARKERS = ("prefill", "pf_", "gemm_kernel<")
 
 
 def _is_frame_end(n):

@@ -41,6 +41,7 @@ def test_prof_summary_names_and_frames():
 
     n = "void sk::(anonymous namespace)::attn_o_kernel<2, 2048, 1, sk::WF32>(sk::GemvArgs, sk::AttnArgs)"
     assert short_name(n) == "attn_o_kernel<2, 2048, 1, sk::WF32>"
-    names = ["gemm_nt_kernel<0>", "final_norm_kernel", "a", "b", "final_norm_kernel", "a", "b",
-             "final_norm_kernel", "a"]
-    assert _frames(names) == [(1, 4), (4, 7)]
+    names = ["final_norm_kernel", "sk::gemm_kernel<0, WF32, 64, 64, 2, 2, 3, 1>", "final_norm_kernel", "a", "b",
+             "final_norm_kernel", "a", "b", "final_norm_kernel", "a"]
+    assert _frames(names) == [(2, 5), (5, 8)]
+    assert _frames([n.replace("sk::gemm_kernel<0, WF32, 64, 64, 2, 2, 3, 1>", "pf_finish_kernel") for n in names]) == [(2, 5), (5, 8)]

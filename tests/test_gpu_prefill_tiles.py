@@ -116,4 +116,5 @@ def test_prefix_alone_in_a_batch_and_as_refill(hip_device, bf16):
     outs.append((e.hidden()[0], _kv(e, 1)[:, 0, :, :38]))
     e.close()
     for hid, kv in outs[1:]:
+        print(f"bf16={bf16}: hidden {_err(hid, outs[0][0]):.2e}, K/V {_err(kv, outs[0][1]):.2e}", flush=True)
         assert _err(hid, outs[0][0]) < (1e-4 if bf16 else 2e-5) and _err(kv, outs[0][1]) < (1e-4 if bf16 else 2e-5)
