@@ -94,16 +94,18 @@ int sk_bind_weight(sk_engine* e, const char* key, const void* dev_ptr, int32_t d
                    const int64_t* shape, int32_t ndim);
 
 /* Stage one row's prefix: text ids, then the frames `frame_codes[n_frames][Q]`
- * (the caller includes the BOS frame first, model.py:633-642).  Resets the row. */
+ * (the caller includes the BOS frame first, model.py:633-642).  Resets the row.
+ * The ids and codes are copied; they are embedded when the prefill runs, with
+ * the weights bound then. */
 int sk_prefill_row(sk_engine* e, int32_t row, const int64_t* text_ids, int32_t n_text,
                    const int64_t* frame_codes, int32_t n_frames);
 /* Run every staged row through the trunk; leaves per-row hidden and KV length.
  * Every row must be staged; the frame counter starts over.  The order of sums
  * (GEMM tiles, K slices, key splits) goes by the tokens of the whole call: a
  * prefix's hidden state and cache can differ in their last bits with what is
- * prefilled beside it, alone, in a batch or as a refill (FP32 weights ~1e-6 of
- * the largest value, BF16 ~1e-5; a BF16 cache rounds such a difference to one
- * place of a few elements).  The same call repeats bit for bit. */
+ * prefilled beside it, alone, in a batch or as a refill (by 2e-6 of the largest
+ * value with FP32 weights, 6e-6 with BF16, where measured; a BF16 cache rounds
+ * such a difference to one place of a few elements).  The same call repeats bit for bit. */
 int sk_prefill_run(sk_engine* e);
 /* sk_prefill_run that allocates no device memory.  No counterpart in the
  * reference: for callers that cannot allocate (serving loops that must not

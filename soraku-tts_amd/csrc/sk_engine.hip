@@ -1530,7 +1530,7 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
     SK_CHECK(ae == hipSuccess, SK_EHIP, "prefill buffers for %d tokens: %s", M, hipGetErrorString(ae));
     bufs = carve_prefill(e->c, e->nqkv, M, e->pf_mem);
   }
-  {
+  auto enqueue = [&]() -> int {
     // in the device's order of engines, like frames: no other engine's frame
     // runs beside the prefill, and prefills of different engines (which share
     // the no-alloc scratch) take turns
@@ -1549,6 +1549,11 @@ static int prefill_staged(sk_engine* e, bool all, bool noalloc) {
       SK_HIP(hipMemsetAsync(e->prefix2, 0, (size_t)R * e->c.d_model * sizeof(float), e->stream));
     }
     SK_HIP(enqueue_batched_prefill(e, M, max_len, bufs));
+    return SK_OK;
+  };
+  if ((rc = enqueue()) != SK_OK) {
+    hipStreamSynchronize(e->stream);   // the table's copy may still read `tab`
+    return rc;
   }
   SK_HIP(hipStreamSynchronize(e->stream));
   for (int r = 0; r < R; ++r)

@@ -187,3 +187,22 @@ for rows, ctx, kv_bf16 in ((6, 256, 0), (6, 257, 0), (8, 640, 0), (8, 513, 1), (
 """)
     got = [int(line.split()[3]) for line in out.splitlines()]
     assert got == [1, 5, 4, 4, 2, 2, 1, 1, 1, 2, 1, 2, 1, 2, 1, 2, 1, 2, 1, 2], out
+
+
+@pytest.mark.parametrize("name,after", [("hipMemsetAsync", 0), ("hipMemsetAsync", 2), ("hipLaunchKernel", 5)])
+def test_failing_prefill_waits_for_its_table(host, name, after):
+    """A prefill that fails after its table's copy was queued waits for the
+    stream: the copy reads host memory that goes away with the call."""
+    host(f"""
+s = TINY
+h = engine(s)
+for r in range(2):
+    assert stage(h, s, r) == 0, error()
+calls()
+stub.stub_fail(b"{name}", {after})
+rc = L.sk_prefill_run(h)
+cs = [c[0] for c in calls()]
+assert rc == _lib.SK_EHIP and "hipMemcpyAsync" in cs and cs[-1] == "hipStreamSynchronize", (rc, cs)
+stub.stub_fail(b"", -1)
+assert L.sk_prefill_run(h) == 0, error()   # the rows are still staged
+""")
