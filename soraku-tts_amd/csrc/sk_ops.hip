@@ -26,15 +26,42 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // A projection of B activation rows.  Up to 4 rows: the GEMV kernels.  More:
 // 32 rows per launch on the FP32 matrix cores (skinny_kernel), where one pass
 // over the weights serves them all (in chunks of 4 rows through the GEMV the
-// weights were read B / 4 times).  us per call, GEMV chunks / one pass: 4 rows,
-// FP32 2051 x 1024 5.2 / 5.6, BF16 2 x 2688 x 1344 8.7 / 11.5; 7 rows 8.5 / 5.6
-// and 14.7 / 11.7, BF16 2 x 6144 x 2048 34 / 18, 2048 x 6144 36 / 15; 20 rows,
-// FP32 2051 x 1024 20 / 7.4.
+// weights are read B / 4 times).  us per launch, GEMV chunks / one pass: 4 rows,
+// FP32 2051 x 1024 4.1 / 4.9; 7 rows BF16 2 x 6144 x 2048 34 / 16.4, 2048 x 6144
+// 36 / 15; 20 rows FP32 2051 x 1024 20 / 7.4.
+//
+// 5 to 8 rows of few but long weight rows (K to 6,144, where measured) keep the
+// two GEMV launches: they spread the rows over the GPU one or two per wave,
+// where the one pass has a workgroup per 16 of them and takes as long as a CU
+// needs to load those and x in 64-byte pieces (16 waves instead of 8 changed
+// nothing).  From 8 KB per output on for 5 and 6 rows (7 and 8: 12 KB FP32, 16
+// KB BF16), up to 1,536 outputs (1,024 of one matrix with K past 3,072) and 24
+// MB of weights, which the second launch finds in cache; not BF16 with a bias,
+// where one pass is faster.  FP32 1024 x 2048, 5 rows 6.5 / 7.6, 1024 x 3072 5
+// rows 7.9 / 10.1, 8 rows 10.9 / 11.1, 512 x 4096 5 rows 8.9 / 12.5, 2 x 1024 x
+// 2048 5 rows 7.9 / 11.8, 8 rows 10.9 / 12.4; BF16 2 x 1024 x 2048 5 rows 8.3 /
+// 9.1, 1024 x 6144 5 rows 11.2 / 13.1.  Past those lines: FP32 2048 x 2048 5
+// rows 10.6 / 8.1, 1024 x 1024 5.5 / 5.0, 2 x 1536 x 3072 8 rows 21.1 / 17.3,
+// BF16 1024 x 2048 8 rows 9 / 5.7.
 constexpr int ROWS_GEMV = 4;
 template <int EPI>
+bool rows_in_chunks(bool bf16, int B, int N, int K) {
+  if (B <= ROWS_GEMV) return true;
+  if (B > 2 * ROWS_GEMV || K > 6144 || (bf16 && EPI == EPI_BIAS)) return false;
+  const size_t row = (size_t)K * (bf16 ? 2 : 4) * (EPI == EPI_SWIGLU ? 2 : 1);
+  const int most = EPI != EPI_SWIGLU && K > 3072 ? 1024 : 1536;
+  return row >= (B <= 6 ? 8192u : bf16 ? 16384u : 12288u) && N <= most && row * N <= (24u << 20);
+}
+template <int EPI>
 int project_rows(hipStream_t st, int wdtype, int B, const GemvArgs& a) {
-  if (B <= ROWS_GEMV) {
-    SK_HIP((launch_gemv<PRO_NONE, EPI>(wdtype, B, a, st)));
+  if (rows_in_chunks<EPI>(wdtype == SK_BF16, B, a.N, a.K)) {
+    for (int b0 = 0; b0 < B; b0 += ROWS_GEMV) {
+      GemvArgs c = a;
+      c.x = a.x + (size_t)b0 * a.ldx;
+      c.out = a.out + (size_t)b0 * a.ldo;
+      if (a.res) c.res = a.res + (size_t)b0 * a.ldr;
+      SK_HIP((launch_gemv<PRO_NONE, EPI>(wdtype, B - b0 < ROWS_GEMV ? B - b0 : ROWS_GEMV, c, st)));
+    }
     return SK_OK;
   }
   for (int b0 = 0; b0 < B; b0 += SK_ROWS) {

@@ -129,7 +129,9 @@ def test_rows_ops_keep_fp32_products(hip_device, B, K, N, bf16):
     got = ops.classifier_gemv(B, N, K)(torch.from_numpy(x).to(hip_device), torch.from_numpy(w).to(hip_device, dt), zero)
     err = np.sqrt(np.mean((got.cpu().numpy() - ref) ** 2) / np.mean(ref ** 2))
     print(f"B={B} K={K} N={N} bf16={bf16}: {err:.2e}", flush=True)
-    assert err < 2e-7   # 24 totals of 32 products: 2^-24 * 0.4 * (sqrt(32 / 2) + sqrt(24 / 2)) = 1.8e-7; measured 1.0e-7 to 1.35e-7
+    # one pass: 24 totals of 32 products, 2^-24 * 0.4 * (sqrt(32 / 2) + sqrt(24 / 2)) = 1.8e-7 (measured 1.0e-7 to
+    # 1.35e-7); 5 rows of long FP32 rows are GEMV launches, 96 products per lane, 2^-24 * 0.4 * sqrt(96) = 2.3e-7
+    assert err < (2.5e-7 if B == 5 and K > 1024 and not bf16 else 2e-7)
 
 
 @pytest.mark.parametrize("B", [5, 16, 17])
@@ -153,3 +155,29 @@ def test_swiglu_workgroup_rule_matches_float64(hip_device, B, K, N, bf16):
                                    *(torch.from_numpy(w).to(hip_device, dt) for w in ws)).cpu().numpy()
     g, u = (x.astype(np.float64) @ w.T.astype(np.float64) for w in ws)
     assert _rel(got, om.silu(g) * u) < 2e-5
+
+
+@pytest.mark.parametrize("B", [5, 6, 7, 8])
+@pytest.mark.parametrize("K,N", [(2040, 96), (2048, 96), (3072, 33), (4096, 48), (6144, 20)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_rows_in_chunks_match_float64(hip_device, B, K, N, bf16):
+    """5 to 8 rows of long weight rows, on both sides of the rule that runs them
+    as two launches of up to 4: every row against float64 (bound as above)."""
+    import torch
+
+    from soraku_amd import ops
+
+    rng = np.random.default_rng(B * 13 + K)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    x, res, bias = (rng.standard_normal(s, dtype=np.float32) for s in ((B, K), (B, N), (N,)))
+    ws = [rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05) for _ in range(2)]
+    ws = [om.round_bf16(w) if bf16 else w for w in ws]
+    print(f"chunks B={B} K={K} N={N} bf16={bf16}", flush=True)
+    xd, wd = torch.from_numpy(x).to(hip_device), [torch.from_numpy(w).to(hip_device, dt) for w in ws]
+    a, b = (x.astype(np.float64) @ w.T.astype(np.float64) for w in ws)
+    got = ops.classifier_gemv(B, N, K)(xd, wd[0], torch.from_numpy(bias).to(hip_device)).cpu().numpy()
+    assert _rel(got, a + bias) < 2e-5
+    got = ops.down_residual_gemv(B, N, K)(xd, wd[0], torch.from_numpy(res).to(hip_device)).cpu().numpy()
+    assert _rel(got, a + res) < 2e-5
+    got = ops.swiglu_gemv(B, N, K)(xd, *wd).cpu().numpy()
+    assert _rel(got, om.silu(a) * b) < 2e-5

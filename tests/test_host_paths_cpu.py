@@ -206,3 +206,30 @@ assert rc == _lib.SK_EHIP and "hipMemcpyAsync" in cs and cs[-1] == "hipStreamSyn
 stub.stub_fail(b"", -1)
 assert L.sk_prefill_run(h) == 0, error()   # the rows are still staged
 """)
+
+
+def test_operator_rows_rule(host):
+    """Which projections of many rows run as GEMV launches of 4 rows and which
+    in one pass of up to 32."""
+    out = host("""
+p = C.c_void_p(4096)
+def run(op, B, N, K, bf16):
+    calls()
+    dt = int(bf16)
+    if op == "bias": rc = L.sk_op_classifier_gemv(None, B, N, K, dt, p, p, p, p)
+    elif op == "resid": rc = L.sk_op_down_residual_gemv(None, B, N, K, dt, p, p, p, p)
+    else: rc = L.sk_op_swiglu_gemv(None, B, N, K, dt, p, p, p, p)
+    assert rc == 0, error()
+    return ["one" if "skinny" in n else "gemv" for n, _ in kernels(calls())]
+for case in (("bias", 4, 1024, 2048, 0), ("bias", 5, 1024, 2048, 0), ("bias", 5, 1024, 2040, 0), ("bias", 7, 1024, 2048, 0),
+             ("resid", 8, 1024, 3072, 0), ("resid", 8, 1536, 3072, 0), ("resid", 5, 1537, 3072, 0), ("resid", 5, 1025, 3080, 0),
+             ("resid", 9, 1024, 3072, 0), ("bias", 5, 1024, 4096, 1), ("resid", 5, 1024, 4096, 1), ("resid", 7, 1024, 6144, 1),
+             ("resid", 5, 16, 6152, 0), ("swiglu", 6, 1024, 1024, 0), ("swiglu", 6, 1536, 2048, 0), ("swiglu", 6, 1536, 2056, 0),
+             ("swiglu", 7, 1024, 4096, 1), ("swiglu", 7, 1024, 4088, 1), ("swiglu", 7, 6144, 2048, 1),
+             ("bias", 20, 2051, 1024, 0), ("bias", 40, 2051, 1024, 0)):
+    print(*case, *run(*case))
+""")
+    g, o = "gemv", "one"
+    want = [[g], [g, g], [o], [o], [g, g], [g, g], [o], [o], [o], [o], [g, g], [o], [o], [g, g], [g, g], [o], [g, g], [o],
+            [o], [o], [o, o]]
+    assert [line.split()[5:] for line in out.splitlines()] == want, out
