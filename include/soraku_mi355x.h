@@ -33,7 +33,8 @@ extern "C" {
 #define SK_ENOWEIGHT  -2   /* a required weight was never bound                           */
 #define SK_ENOCAPTURE -3   /* step before capture (graph_frame.py:301-302)                 */
 #define SK_EKVFULL    -4   /* KV cache or frame ring full (graph_frame.py:155-156)         */
-#define SK_EHIP       -5   /* a HIP runtime call failed; sk_last_error() holds its text    */
+#define SK_EHIP       -5   /* a HIP runtime call failed, or host memory for a prefix ran out;
+                              sk_last_error() says which                                  */
 #define SK_ESTATE     -6   /* call out of order (e.g. step before prefill)                 */
 
 /* ---- element types --------------------------------------------------- */
